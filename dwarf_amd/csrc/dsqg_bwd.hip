@@ -6,6 +6,7 @@
 // (kernels/dsqg_attention_v3.py:265-271), whose summation order varies run to run.
 #include "dsqg_common.hpp"
 #include "dsqg_launch.hpp"
+#include "dsqg_f32.hpp"
 #include "dsqg_reduce.hpp"
 
 namespace dsqg {
@@ -45,10 +46,16 @@ bool bwd_mfma_supported(const BwdParams& p, int D, int dtype) {
          rmin >= D && span < (1LL << 31);
 }
 
+bool bwd_f32_supported(const BwdParams& p, int D, int dtype) {
+  const long long rs[4] = {p.qs.n, p.ks.n, p.vs.n, p.dos.n};
+  return dtype == 0 && f32_mfma_strides_ok(p.N, p.taps.maxd, D, rs, 4);
+}
+
 void bwd_plan(BwdParams& p, int D, int dtype, bool se) {
   const bool mfma = bwd_mfma_supported(p, D, dtype);
-  const int QPB = mfma ? 64 : kBlock / lanes_per_row(D);  // dq rows per tile
-  const int KPB = mfma ? 64 : kBlock / lanes_per_row(D);  // dk/dv rows per workgroup
+  const bool tile64 = mfma || bwd_f32_supported(p, D, dtype);
+  const int QPB = tile64 ? 64 : kBlock / lanes_per_row(D);  // dq rows per tile
+  const int KPB = tile64 ? 64 : kBlock / lanes_per_row(D);  // dk/dv rows per workgroup
   p.n_tiles = (p.N + QPB - 1) / QPB;
   p.n_tiles_kv = (p.N + KPB - 1) / KPB;
   // One tile per workgroup: the partial rows (J floats) are small next to a tile's loads, and the

@@ -1,4 +1,4 @@
-// DSQG backward, launch 2: key-centric dk/dv (VALU path, fp32 and bf16).
+// DSQG backward, launch 2: key-centric dk/dv (VALU path, see dsqg_fwd.hip).
 //
 // Key row m gathers the queries n = m + delta_j that read it:
 //   dv_m = sum_j a alpha_j(n) dOut_n,   dk_m = c sum_j g_j dS_j(n) q_n,
@@ -161,6 +161,7 @@ static hipError_t launch_bwd_dkdv_dtype(const BwdParams& p, int D, unsigned nb, 
 
 hipError_t launch_bwd_dkdv(const BwdParams& p, int dtype, int D, unsigned nblocks, hipStream_t st) {
   if (bwd_mfma_supported(p, D, dtype)) return launch_bwd_dkdv_mfma(p, D, nblocks, st);
+  if (bwd_f32_supported(p, D, dtype)) return launch_bwd_dkdv_f32(p, D, nblocks, st);
   return dtype == 0 ? launch_bwd_dkdv_dtype<float>(p, D, nblocks, st) : hipErrorNotSupported;
 }
 

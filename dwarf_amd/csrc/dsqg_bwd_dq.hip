@@ -1,4 +1,5 @@
-// DSQG backward, VALU path (fp32 and bf16).  Three launches, no global atomics
+// DSQG backward, VALU path: the float32 calls dsqg_bwd_dq_f32.hip's 32-bit row offsets do not
+// reach (see dsqg_fwd.hip).  Three launches, no global atomics
 // (this file: launch 1; dsqg_bwd_dkdv.hip: launch 2; dsqg_bwd.hip: launch 3 and the driver):
 //
 //  1. bwd_dq_kernel (query-centric).  Per query row n: recompute s_j and alpha_j = exp(s_j - lse)
@@ -249,6 +250,7 @@ static hipError_t launch_bwd_dq_dtype(const BwdParams& p, int D, unsigned nb, hi
 
 hipError_t launch_bwd_dq(const BwdParams& p, int dtype, int D, unsigned nblocks, hipStream_t st) {
   if (bwd_mfma_supported(p, D, dtype)) return launch_bwd_dq_mfma(p, D, nblocks, st);
+  if (bwd_f32_supported(p, D, dtype)) return launch_bwd_dq_f32(p, D, nblocks, st);
   return dtype == 0 ? launch_bwd_dq_dtype<float>(p, D, nblocks, st) : hipErrorNotSupported;
 }
 

@@ -1,5 +1,5 @@
-// DSQG forward, VALU path: fp32, and bf16 offset tables outside the MFMA kernel's reach
-// (more than kMaxSparse taps beyond the dense window).
+// DSQG forward, VALU path: the float32 calls whose strides dsqg_fwd_f32.hip's 32-bit row offsets
+// do not reach (slices of 2 GiB and more, rows that overlap); it addresses with 64 bits.
 //
 // One workgroup = one (b,h) and a tile of QPB query rows.  Each query row is owned by a group
 // of G consecutive lanes (D/8 rounded up to a power of two), lane g holding elements
@@ -174,9 +174,10 @@ static hipError_t launch_fwd_dtype(const FwdParams& p, int D, hipStream_t st) {
 }
 
 hipError_t launch_fwd(const FwdParams& p, int dtype, int D, hipStream_t st) {
-  // fp32 runs these VALU kernels; bf16 runs only the MFMA kernel (the ABI rejects a bf16 call
-  // it cannot take with DSQG_EUNSUPPORTED before getting here).
-  if (dtype == 0) return launch_fwd_dtype<float>(p, D, st);
+  // fp32 runs the float32 MFMA kernel, or these VALU kernels where its 32-bit row offsets do not
+  // reach; bf16 runs only the MFMA kernel (the ABI rejects a bf16 call it cannot take with
+  // DSQG_EUNSUPPORTED before getting here).
+  if (dtype == 0) return fwd_f32_supported(p, D) ? launch_fwd_f32(p, D, st) : launch_fwd_dtype<float>(p, D, st);
   if (fwd_mfma_supported(p, D)) return launch_fwd_mfma(p, D, st);
   return hipErrorNotSupported;
 }

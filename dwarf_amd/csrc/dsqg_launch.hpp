@@ -15,6 +15,14 @@ hipError_t launch_fwd(const FwdParams& p, int dtype, int D, hipStream_t st);
 bool fwd_mfma_supported(const FwdParams& p, int D);
 hipError_t launch_fwd_mfma(const FwdParams& p, int D, hipStream_t st);
 
+// float32 MFMA kernels (dsqg_*_f32.hip): row strides >= D and 32-bit byte offsets within each
+// (b,h) slice.  The launchers below take the VALU kernels for any other float32 call.
+bool fwd_f32_supported(const FwdParams& p, int D);
+hipError_t launch_fwd_f32(const FwdParams& p, int D, hipStream_t st);
+bool bwd_f32_supported(const BwdParams& p, int D, int dtype);
+hipError_t launch_bwd_dq_f32(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
+hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
+
 // Tiling of the backward for these sizes and kernel choice; fills n_tiles / tiles_per_block /
 // n_chunks / n_tiles_kv (se: scale_embed or its gradient is present).
 void bwd_plan(BwdParams& p, int D, int dtype, bool se);
