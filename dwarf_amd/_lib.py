@@ -117,6 +117,7 @@ SIGNATURES = {
 }
 
 _LIB = None
+_HOST = None
 
 
 class DSQGLibraryError(RuntimeError):
@@ -142,6 +143,25 @@ def load() -> ctypes.CDLL:
         raise DSQGLibraryError(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}")
     _LIB = lib
     return lib
+
+
+def host():
+    """The native host layer (_dsqg_host.so) bound to the library of ``load()``; raise if it is
+    missing."""
+    global _HOST
+    if _HOST is not None:
+        return _HOST
+    lib = load()
+    try:
+        from . import _dsqg_host as mod
+    except ImportError as e:
+        raise DSQGLibraryError(
+            f"the native host layer {PKG_DIR / '_dsqg_host.so'} does not load ({e}): build it with "
+            "`python -m dwarf_amd.build`") from e
+    mod.init({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES},
+             DSQGLibraryError)
+    _HOST = mod
+    return mod
 
 
 def status_string(code: int) -> str:

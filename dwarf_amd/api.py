@@ -30,7 +30,7 @@ from typing import Optional, Sequence
 import torch
 from torch import Tensor
 
-from . import ops
+from . import _lib, ops
 from .offsets import default_offsets, validate
 
 
@@ -71,13 +71,17 @@ def dsqg_attention(q: Tensor, k: Tensor, v: Tensor, pos_bias: Tensor,
     q, k, v [B,H,N,HD]; pos_bias [J,H]; scale_embed [J,HD]; score_gain [H,J]; if_gain [H].
     Differentiable in q, k, v and every parameter.
     """
+    if not ops.traced(q, k, v):
+        return _lib.host().attention(q, k, v, pos_bias, scale_embed, score_gain, if_gain,
+                                     default_offsets(pos_bias.shape[0]) if offsets is None
+                                     else offsets)[0]
     offs = validate(offsets) if offsets is not None else default_offsets(pos_bias.shape[0])
     _check_shapes(q, k, v, pos_bias, scale_embed, score_gain, if_gain, offs)
     orig = q.dtype
     q, k, v = _compute_dtype(q, k, v)
     args = (q, k, v, pos_bias.float(), _f32(scale_embed), _f32(score_gain), _f32(if_gain),
             list(offs))
-    out = (ops.dsqg_fwd(*args) if ops.traced(q, k, v) else ops.AttentionFn.apply(*args))[0]
+    out = ops.dsqg_fwd(*args)[0]
     return out if out.dtype == orig else out.to(orig)
 
 
@@ -95,6 +99,11 @@ def dsqg_attention_qkv(qkv: Tensor, num_heads: int, pos_bias: Tensor,
     train/train_2048_condU.py:178-181); the deltas' gradients are the K / V slices of d(qkv).
     """
     assert qkv.dim() == 3, f"qkv must be [B,N,3*H*HD], got {tuple(qkv.shape)}"
+    k_delta, v_delta = (None, None) if kv_inject is None else kv_inject
+    if not ops.traced(qkv, *(() if kv_inject is None else (k_delta, v_delta))):
+        return _lib.host().attention_qkv(qkv, num_heads, pos_bias, scale_embed, score_gain, if_gain,
+                                         default_offsets(pos_bias.shape[0]) if offsets is None
+                                         else offsets, k_delta, v_delta)
     offs = validate(offsets) if offsets is not None else default_offsets(pos_bias.shape[0])
     q, k, v = ops.split_qkv(qkv, num_heads)
     _check_shapes(q, k, v, pos_bias, scale_embed, score_gain, if_gain, offs)
@@ -103,15 +112,11 @@ def dsqg_attention_qkv(qkv: Tensor, num_heads: int, pos_bias: Tensor,
         qkv = qkv.bfloat16()
     params = (pos_bias.float(), _f32(scale_embed), _f32(score_gain), _f32(if_gain), list(offs))
     if kv_inject is None:
-        args = (qkv, num_heads, *params)
-        out = (ops.dsqg_fwd_qkv(*args) if ops.traced(qkv) else ops.AttentionQkvFn.apply(*args))[0]
+        out = ops.dsqg_fwd_qkv(qkv, num_heads, *params)[0]
     else:
-        k_delta, v_delta = kv_inject
         assert k_delta.shape == k.shape and v_delta.shape == v.shape, \
             f"kv_inject deltas must be {tuple(k.shape)}"
-        args = (qkv, k_delta, v_delta, num_heads, *params)
-        fn = ops.dsqg_fwd_qkv_kv if ops.traced(qkv, k_delta, v_delta) else ops.AttentionQkvKvFn.apply
-        out = fn(*args)[0]
+        out = ops.dsqg_fwd_qkv_kv(qkv, k_delta, v_delta, num_heads, *params)[0]
     return out if out.dtype == orig else out.to(orig)
 
 
@@ -135,13 +140,17 @@ def dsqg_attention_backend(q: Tensor, k: Tensor, v: Tensor, pos_bias: Tensor,
 def dsqg_attention_with_lse(q, k, v, pos_bias, scale_embed=None, *, offsets=None,
                             score_gain=None, if_gain=None):
     """(out, lse): out in the dtype rules above (differentiable), lse [B,H,N] fp32 (not)."""
+    if not ops.traced(q, k, v):
+        return _lib.host().attention(q, k, v, pos_bias, scale_embed, score_gain, if_gain,
+                                     default_offsets(pos_bias.shape[0]) if offsets is None
+                                     else offsets)
     offs = validate(offsets) if offsets is not None else default_offsets(pos_bias.shape[0])
     _check_shapes(q, k, v, pos_bias, scale_embed, score_gain, if_gain, offs)
     orig = q.dtype
     q, k, v = _compute_dtype(q, k, v)
     args = (q, k, v, pos_bias.float(), _f32(scale_embed), _f32(score_gain), _f32(if_gain),
             list(offs))
-    out, lse = (ops.dsqg_fwd(*args) if ops.traced(q, k, v) else ops.AttentionFn.apply(*args))[:2]
+    out, lse = ops.dsqg_fwd(*args)[:2]
     return (out if out.dtype == orig else out.to(orig)), lse
 
 
@@ -151,6 +160,11 @@ def dsqg_decode_step(q: Tensor, k_new: Tensor, v_new: Tensor, k_ring: Tensor, v_
                      score_gain: Optional[Tensor] = None,
                      if_gain: Optional[Tensor] = None) -> Tensor:
     """One decode step: q/k_new/v_new [B,H,D], rings [B,H,S,D] (updated in place), pos [B]."""
+    rows = (q, k_new, v_new, k_ring, v_ring)
+    # (The step has no gradient; the custom op is what says so when one is asked for.)
+    if not ops.traced(*rows, pos) and not (torch.is_grad_enabled() and any(t.requires_grad for t in rows)):
+        return _lib.host().decode(*rows, pos, pos_bias, scale_embed, score_gain, if_gain,
+                                  default_offsets(pos_bias.shape[0]) if offsets is None else offsets)
     offs = validate(offsets) if offsets is not None else default_offsets(pos_bias.shape[0])
 
     def f32(t):
@@ -177,7 +191,7 @@ def causal_mean_pool_gate(x: Tensor, gate_pre: Tensor) -> Tensor:
     assert x.shape[2] % 8 == 0, f"channel count {x.shape[2]} must be a multiple of 8"
     if ops.traced(x, gate_pre):
         return ops.pool_gate_fwd(x, gate_pre)
-    return ops.PoolGateFn.apply(x, gate_pre)
+    return _lib.host().pool_gate(x, gate_pre)
 
 
 class DSQGRingCache:

@@ -1,7 +1,9 @@
-"""Build libdsqg_hip.so (the C-ABI HIP library) in-tree for gfx950.
+"""Build libdsqg_hip.so (the C-ABI HIP library) and _dsqg_host.so (the native host layer of the
+eager public functions) in-tree for gfx950.
 
 Each ``csrc/*.hip`` file is compiled to an object by its own ``hipcc`` process (in parallel),
-then the objects are linked into ``dwarf_amd/libdsqg_hip.so``.  Usage:
+then the objects are linked into ``dwarf_amd/libdsqg_hip.so``; ``csrc/dsqg_host.cpp`` is compiled
+by the host compiler against torch's headers into ``dwarf_amd/_dsqg_host.so``.  Usage:
 
     python -m dwarf_amd.build            # build (always recompiles)
     python -m dwarf_amd.build --jobs 4
@@ -23,6 +25,7 @@ CSRC = PKG_DIR / "csrc"
 INCLUDE = PKG_DIR.parent / "include"
 LIB_NAME = "libdsqg_hip.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+HOST_PATH = PKG_DIR / "_dsqg_host.so"
 OBJ_DIR = PKG_DIR / "_build"
 
 ARCH = "gfx950"
@@ -62,17 +65,43 @@ def _compile(src: Path, hipcc: str) -> tuple[Path, float, str]:
     return obj, time.time() - t0, log
 
 
+def _build_host(hipcc: str) -> tuple[Path, float, str]:
+    """Compile csrc/dsqg_host.cpp (host code only) into _dsqg_host.so."""
+    import sysconfig
+    import torch
+    t0 = time.time()
+    troot = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc).resolve().parents[1]
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-I{troot}/include", f"-I{troot}/include/torch/csrc/api/include",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{rocm}/include",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_dsqg_host",
+           "-DTORCH_API_INCLUDE_EXTENSION_H",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           str(CSRC / "dsqg_host.cpp"), "-o", str(tmp), f"-L{troot}/lib",
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host compile failed:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH, time.time() - t0, ""
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> Path:
-    """Compile every csrc/*.hip for gfx950 and link libdsqg_hip.so; returns its path."""
+    """Compile every csrc/*.hip for gfx950 and link libdsqg_hip.so, and the host layer beside it;
+    returns the library's path."""
     hipcc = hipcc_path()
     OBJ_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
-    jobs = jobs or min(len(sources), max(1, (os.cpu_count() or 2)))
+    jobs = jobs or min(len(sources) + 1, max(1, (os.cpu_count() or 2)))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host, hipcc)
         results = list(ex.map(lambda s: _compile(s, hipcc), sources))
-    for obj, dt, log in results:
+        host = host.result()
+    for obj, dt, log in results + [host]:
         if verbose:
             print(f"[dwarf_amd.build] {obj.name}: {dt:.1f}s", flush=True)
             if log:

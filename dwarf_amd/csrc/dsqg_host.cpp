@@ -1,0 +1,563 @@
+// Native host layer of the eager public functions (dwarf_amd/api.py): argument checks, the C ABI's
+// argument blocks, output and workspace allocation and autograd, in C++.
+//
+// The kernels of a training step take a few tens to two hundred microseconds; the same steps
+// through Python objects (ctypes blocks, a Python autograd function whose backward runs on the
+// engine's thread) took 220-350 us of host time per forward + backward on the MI355X host, and
+// bounded every call but the largest.  Traced code (torch.compile, export, fake tensors) sees the
+// custom ops of dwarf_amd/ops.py instead.
+//
+// The entry points of libdsqg_hip.so arrive as addresses from the loader (dwarf_amd/_lib.py), so
+// the library that was checked there is the one called here.  Nothing is kept between calls.
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include <array>
+#include <optional>
+
+#include "../../include/dsqg.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+namespace {
+
+struct Api {
+  decltype(&dsqg_status_string) status_string = nullptr;
+  decltype(&dsqg_fwd) fwd = nullptr;
+  decltype(&dsqg_bwd_workspace_size) bwd_workspace_size = nullptr;
+  decltype(&dsqg_bwd) bwd = nullptr;
+  decltype(&dsqg_decode_step) decode_step = nullptr;
+  decltype(&dsqg_pool_gate_workspace_size) pool_workspace_size = nullptr;
+  decltype(&dsqg_pool_gate_fwd) pool_fwd = nullptr;
+  decltype(&dsqg_pool_gate_bwd) pool_bwd = nullptr;
+  PyObject* library_error = nullptr;  // dwarf_amd._lib.DSQGLibraryError
+} api;
+
+// ---- Errors (Python exceptions; the backward runs without the GIL). --------------------------
+
+[[noreturn]] void raise(PyObject* type, const std::string& msg) {
+  py::gil_scoped_acquire gil;
+  PyErr_SetString(type, msg.c_str());
+  throw py::error_already_set();
+}
+
+template <typename... A>
+void require(bool ok, const A&... msg) {
+  if (!ok) raise(PyExc_AssertionError, c10::str(msg...));
+}
+
+void check(int status, const char* what) {
+  if (status != DSQG_OK)
+    raise(api.library_error, c10::str(what, " failed: status ", status, " (", api.status_string(status), ")"));
+}
+
+// Python's spelling of a shape, for the assertion messages.
+std::string shape_str(c10::IntArrayRef s) {
+  std::string r = "(";
+  for (size_t i = 0; i < s.size(); ++i) r += (i ? ", " : "") + std::to_string(s[i]);
+  return r + (s.size() == 1 ? ",)" : ")");
+}
+
+c10::Device require_gpu(std::initializer_list<const Tensor*> ts) {
+  std::optional<c10::Device> dev;
+  for (const Tensor* t : ts) {
+    if (!t->defined()) continue;
+    if (!t->is_cuda())
+      raise(PyExc_RuntimeError, c10::str("dwarf_amd DSQG ops need tensors on a ROCm GPU, got device ", t->device(),
+                                         "; there is no CPU implementation"));
+    if (!dev) dev = t->device();
+    else if (*dev != t->device())
+      raise(PyExc_RuntimeError, c10::str("tensors on different devices: ", *dev, " and ", t->device()));
+  }
+  return *dev;
+}
+
+dsqg_stream_t stream_of(const c10::Device& dev) {
+  return reinterpret_cast<dsqg_stream_t>(c10::hip::getCurrentHIPStream(dev.index()).stream());
+}
+
+// ---- Offset tables. ----------------------------------------------------------------------------
+
+struct Table : torch::CustomClassHolder {
+  int J = 0;
+  int NS = 0;  // taps beyond the dense window 0, 1, .., W (W <= 32)
+  int32_t offsets[DSQG_MAX_OFFSETS] = {};
+};
+using TablePtr = c10::intrusive_ptr<Table>;
+
+// A sequence of ints, strictly increasing from 0 (offsets.validate's rule and message).
+TablePtr make_table(const py::object& seq) {
+  TablePtr t = c10::make_intrusive<Table>();
+  std::vector<long long> v;
+  for (const py::handle& item : seq) {
+    if (PyLong_CheckExact(item.ptr())) v.push_back(item.cast<long long>());
+    else v.push_back(py::int_(py::reinterpret_borrow<py::object>(item)).cast<long long>());
+  }
+  bool ok = !v.empty() && v[0] == 0;
+  for (size_t j = 1; ok && j < v.size(); ++j) ok = v[j] > v[j - 1];
+  if (!ok) {
+    py::tuple offs(v.size());
+    for (size_t j = 0; j < v.size(); ++j) offs[j] = v[j];
+    raise(PyExc_AssertionError, "offsets must be strictly increasing and start at 0: " + py::str(offs).cast<std::string>());
+  }
+  if (v.size() > DSQG_MAX_OFFSETS)
+    raise(PyExc_ValueError, c10::str("offset table must have 1..", DSQG_MAX_OFFSETS, " entries, got ", v.size()));
+  t->J = (int)v.size();
+  for (int j = 0; j < t->J; ++j)
+    t->offsets[j] = (int32_t)std::min<long long>(v[j], std::numeric_limits<int32_t>::max());
+  int W = 0;
+  while (W + 1 < t->J && W + 1 <= 32 && t->offsets[W + 1] == W + 1) ++W;
+  t->NS = t->J - W - 1;
+  return t;
+}
+
+void fill_shape(dsqg_shape& s, at::ScalarType dt, int64_t B, int64_t H, int64_t N, int64_t D, const Table& t) {
+  s.dtype = dt == at::kFloat ? DSQG_F32 : DSQG_BF16;
+  s.B = (int32_t)B; s.H = (int32_t)H; s.N = (int32_t)N; s.D = (int32_t)D; s.J = t.J;
+  std::copy(std::begin(t.offsets), std::end(t.offsets), s.offsets);
+}
+
+// ---- Tensors as the kernels take them. -----------------------------------------------------------
+
+void* ptr(const Tensor& t) { return !t.defined() || t.numel() == 0 ? nullptr : t.data_ptr(); }
+
+// t if the kernels can read it in place (unit inner stride, 16-byte aligned rows), else a copy.
+Tensor rows_ready(const Tensor& t) {
+  if (t.numel() == 0) return t;
+  const int64_t es = t.element_size(), d = t.dim();
+  bool ok = t.stride(d - 1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  for (int64_t i = 0; ok && i < d - 1; ++i) ok = t.stride(i) >= 0 && (t.stride(i) * es) % 16 == 0;
+  return ok ? t : t.contiguous();
+}
+
+// fp32, contiguous and 16-byte aligned (the kernels read scale_embed as 16-byte pieces).
+Tensor param(const Tensor& t) {
+  if (!t.defined()) return t;
+  if (t.scalar_type() == at::kFloat && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0)
+    return t;
+  return t.detach().to(at::kFloat).clone(at::MemoryFormat::Contiguous);
+}
+
+void set_strides(int64_t (&dst)[4], const Tensor& t) {
+  for (int i = 0; i < 4; ++i) dst[i] = t.stride(i);
+}
+
+// One of q, k, v (part 0, 1, 2) as a [B,H,N,HD] view of qkv [B,N,3*H*HD].
+Tensor head_view(const Tensor& qkv, int64_t H, int64_t part) {
+  const int64_t E = qkv.size(2) / 3, HD = E / H, sc = qkv.stride(2);
+  return qkv.as_strided({qkv.size(0), H, qkv.size(1), HD}, {qkv.stride(0), HD * sc, qkv.stride(1), sc},
+                        qkv.storage_offset() + part * E * sc);
+}
+
+struct Params {
+  Tensor pb, se, sg, ig;  // undefined when absent
+};
+
+// ---- Forward. --------------------------------------------------------------------------------------
+
+struct FwdOut {
+  Tensor out, lse, alpha_lr;
+};
+
+FwdOut run_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Params& P, const Table& t) {
+  const c10::Device dev = require_gpu({&q0, &k0, &v0, &P.pb, &P.se, &P.sg, &P.ig});
+  const auto dt = q0.scalar_type();
+  require((dt == at::kFloat || dt == at::kBFloat16) && k0.scalar_type() == dt && v0.scalar_type() == dt,
+          "q/k/v must share dtype float32 or bfloat16, got ", dt, "/", k0.scalar_type(), "/", v0.scalar_type());
+  const c10::OptionalDeviceGuard guard(dev);
+  const int64_t B = q0.size(0), H = q0.size(1), N = q0.size(2), D = q0.size(3);
+  const Tensor q = rows_ready(q0), k = rows_ready(k0), v = rows_ready(v0);
+  const Tensor pb = param(P.pb), se = param(P.se), sg = param(P.sg), ig = param(P.ig);
+  const auto f32 = q.options().dtype(at::kFloat);
+  FwdOut r;
+  // Token-major storage: the callers' head merge is a view.
+  r.out = at::empty_strided({B, H, N, D}, {N * H * D, D, H * D, 1}, q.options());
+  r.lse = at::empty({B, H, N}, f32);
+  if (dt == at::kBFloat16 && t.NS > 0) r.alpha_lr = at::empty({B, H, t.NS, N}, f32);
+  else r.alpha_lr = at::empty({0}, f32);
+  dsqg_fwd_args a = {};
+  fill_shape(a.shape, dt, B, H, N, D, t);
+  a.q = ptr(q); set_strides(a.q_stride, q);
+  a.k = ptr(k); set_strides(a.k_stride, k);
+  a.v = ptr(v); set_strides(a.v_stride, v);
+  a.pos_bias = static_cast<const float*>(ptr(pb));
+  a.scale_embed = static_cast<const float*>(ptr(se));
+  a.score_gain = static_cast<const float*>(ptr(sg));
+  a.if_gain = static_cast<const float*>(ptr(ig));
+  a.out = ptr(r.out); set_strides(a.out_stride, r.out);
+  a.lse = static_cast<float*>(ptr(r.lse));
+  a.alpha_lr = static_cast<float*>(ptr(r.alpha_lr));
+  check(api.fwd(&a, stream_of(dev)), "dsqg_fwd");
+  return r;
+}
+
+// ---- Backward. ---------------------------------------------------------------------------------------
+
+struct Grads {
+  Tensor dq, dk, dv, dpb, dse, dsg, dig;  // dq, dk, dv allocated by the caller or here
+};
+
+void run_bwd(Grads& G, const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& dout0, const Tensor& lse0,
+             const Tensor& alpha0, const Params& P, const Table& t, bool need_dse, bool need_dsg, bool need_dig) {
+  const c10::Device dev = require_gpu({&q0, &k0, &v0, &dout0, &lse0, &P.pb, &P.se, &P.sg, &P.ig});
+  const c10::OptionalDeviceGuard guard(dev);
+  const auto dt = q0.scalar_type();
+  const int64_t B = q0.size(0), H = q0.size(1), N = q0.size(2), D = q0.size(3);
+  const Tensor q = rows_ready(q0), k = rows_ready(k0), v = rows_ready(v0), dout = rows_ready(dout0.to(dt));
+  const Tensor lse = lse0.contiguous(), alpha = alpha0.contiguous();
+  const Tensor pb = param(P.pb), se = param(P.se), sg = param(P.sg), ig = param(P.ig);
+  const auto f32 = q.options().dtype(at::kFloat);
+  if (!G.dq.defined()) {
+    G.dq = at::empty({B, H, N, D}, q.options());
+    G.dk = at::empty({B, H, N, D}, q.options());
+    G.dv = at::empty({B, H, N, D}, q.options());
+  }
+  G.dpb = at::empty({t.J, H}, f32);
+  if (need_dse) G.dse = at::empty({t.J, D}, f32);
+  if (need_dsg) G.dsg = at::empty({H, t.J}, f32);
+  if (need_dig) G.dig = at::empty({H}, f32);
+  dsqg_bwd_args a = {};
+  fill_shape(a.shape, dt, B, H, N, D, t);
+  a.q = ptr(q); set_strides(a.q_stride, q);
+  a.k = ptr(k); set_strides(a.k_stride, k);
+  a.v = ptr(v); set_strides(a.v_stride, v);
+  a.dout = ptr(dout); set_strides(a.dout_stride, dout);
+  a.lse = static_cast<const float*>(ptr(lse));
+  a.alpha_lr = static_cast<const float*>(ptr(alpha));
+  a.pos_bias = static_cast<const float*>(ptr(pb));
+  a.scale_embed = static_cast<const float*>(ptr(se));
+  a.score_gain = static_cast<const float*>(ptr(sg));
+  a.if_gain = static_cast<const float*>(ptr(ig));
+  a.dq = ptr(G.dq); set_strides(a.dq_stride, G.dq);
+  a.dk = ptr(G.dk); set_strides(a.dk_stride, G.dk);
+  a.dv = ptr(G.dv); set_strides(a.dv_stride, G.dv);
+  a.dpos_bias = static_cast<float*>(ptr(G.dpb));
+  a.dscale_embed = static_cast<float*>(ptr(G.dse));
+  a.dscore_gain = static_cast<float*>(ptr(G.dsg));
+  a.dif_gain = static_cast<float*>(ptr(G.dig));
+  size_t nbytes = 0;
+  check(api.bwd_workspace_size(&a, &nbytes), "dsqg_bwd_workspace_size");
+  const Tensor ws = at::empty({std::max<int64_t>((int64_t)nbytes, 1)}, q.options().dtype(at::kByte));
+  a.workspace = ws.data_ptr();
+  a.workspace_bytes = nbytes;
+  check(api.bwd(&a, stream_of(dev)), "dsqg_bwd");
+}
+
+// ---- Autograd. ------------------------------------------------------------------------------------------
+
+// Which of an autograd function's arguments, in their order, need a gradient (absent ones do not;
+// the context counts only the tensors that are there).
+struct Needs {
+  std::array<bool, 8> need{};
+  Needs(AutogradContext* ctx, std::initializer_list<bool> present) {
+    size_t edge = 0, i = 0;
+    for (bool p : present) need[i++] = p && ctx->needs_input_grad(edge++);
+  }
+};
+
+OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; }
+Tensor undef(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+Table& table_of(AutogradContext* ctx) {
+  return *c10::static_intrusive_pointer_cast<Table>(ctx->saved_data["table"].toCapsule());
+}
+
+struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                               const Tensor& pb, const OptTensor& se, const OptTensor& sg, const OptTensor& ig,
+                               const TablePtr& t) {
+    const FwdOut r = run_fwd(q, k, v, {pb, undef(se), undef(sg), undef(ig)}, *t);
+    ctx->save_for_backward({q, k, v, r.lse, r.alpha_lr, pb, undef(se), undef(sg), undef(ig)});
+    ctx->saved_data["table"] = c10::IValue::make_capsule(t);
+    ctx->mark_non_differentiable({r.lse, r.alpha_lr});
+    return {r.out, r.lse, r.alpha_lr};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const variable_list s = ctx->get_saved_variables();
+    const Params P{s[5], s[6], s[7], s[8]};
+    const Needs n(ctx, {true, true, true, true, P.se.defined(), P.sg.defined(), P.ig.defined()});
+    Grads G;
+    run_bwd(G, s[0], s[1], s[2], g[0], s[3], s[4], P, table_of(ctx), n.need[4], n.need[5], n.need[6]);
+    return {G.dq, G.dk, G.dv, G.dpb, G.dse, G.dsg, G.dig, Tensor()};
+  }
+};
+
+// q, k, v as the head views of one projection output; its gradient is one tensor.
+struct AttentionQkvFunction : torch::autograd::Function<AttentionQkvFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& pb, const OptTensor& se,
+                               const OptTensor& sg, const OptTensor& ig, int64_t H, const TablePtr& t) {
+    const FwdOut r = run_fwd(head_view(qkv, H, 0), head_view(qkv, H, 1), head_view(qkv, H, 2),
+                             {pb, undef(se), undef(sg), undef(ig)}, *t);
+    ctx->save_for_backward({qkv, r.lse, r.alpha_lr, pb, undef(se), undef(sg), undef(ig)});
+    ctx->saved_data["table"] = c10::IValue::make_capsule(t);
+    ctx->saved_data["H"] = H;
+    ctx->mark_non_differentiable({r.lse, r.alpha_lr});
+    return {r.out, r.lse, r.alpha_lr};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const variable_list s = ctx->get_saved_variables();
+    const int64_t H = ctx->saved_data["H"].toInt();
+    const Params P{s[3], s[4], s[5], s[6]};
+    const Needs n(ctx, {true, true, P.se.defined(), P.sg.defined(), P.ig.defined()});
+    const Tensor dqkv = at::empty_like(s[0], at::MemoryFormat::Contiguous);
+    Grads G;
+    G.dq = head_view(dqkv, H, 0); G.dk = head_view(dqkv, H, 1); G.dv = head_view(dqkv, H, 2);
+    run_bwd(G, head_view(s[0], H, 0), head_view(s[0], H, 1), head_view(s[0], H, 2), g[0], s[1], s[2], P,
+            table_of(ctx), n.need[2], n.need[3], n.need[4]);
+    return {dqkv, G.dpb, G.dse, G.dsg, G.dig, Tensor(), Tensor()};
+  }
+};
+
+// The same with a K/V injection: K + k_delta and V + v_delta are attended, and the K and V slices
+// of d(qkv) are also the deltas' gradients.
+struct AttentionQkvKvFunction : torch::autograd::Function<AttentionQkvKvFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& kd, const Tensor& vd,
+                               const Tensor& pb, const OptTensor& se, const OptTensor& sg, const OptTensor& ig,
+                               int64_t H, const TablePtr& t) {
+    const auto dt = qkv.scalar_type();
+    const Tensor k = head_view(qkv, H, 1) + kd.to(dt), v = head_view(qkv, H, 2) + vd.to(dt);
+    const FwdOut r = run_fwd(head_view(qkv, H, 0), k, v, {pb, undef(se), undef(sg), undef(ig)}, *t);
+    ctx->save_for_backward({qkv, k, v, r.lse, r.alpha_lr, pb, undef(se), undef(sg), undef(ig)});
+    ctx->saved_data["table"] = c10::IValue::make_capsule(t);
+    ctx->saved_data["H"] = H;
+    ctx->saved_data["kd"] = (int64_t)kd.scalar_type();
+    ctx->saved_data["vd"] = (int64_t)vd.scalar_type();
+    ctx->mark_non_differentiable({r.lse, r.alpha_lr, k, v});
+    return {r.out, r.lse, r.alpha_lr, k, v};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const variable_list s = ctx->get_saved_variables();
+    const int64_t H = ctx->saved_data["H"].toInt();
+    const Params P{s[5], s[6], s[7], s[8]};
+    const Needs n(ctx, {true, true, true, true, P.se.defined(), P.sg.defined(), P.ig.defined()});
+    const Tensor dqkv = at::empty_like(s[0], at::MemoryFormat::Contiguous);
+    Grads G;
+    G.dq = head_view(dqkv, H, 0); G.dk = head_view(dqkv, H, 1); G.dv = head_view(dqkv, H, 2);
+    run_bwd(G, head_view(s[0], H, 0), s[1], s[2], g[0], s[3], s[4], P, table_of(ctx), n.need[4], n.need[5],
+            n.need[6]);
+    return {dqkv, G.dk.to((at::ScalarType)ctx->saved_data["kd"].toInt()),
+            G.dv.to((at::ScalarType)ctx->saved_data["vd"].toInt()), G.dpb, G.dse, G.dsg, G.dig, Tensor(), Tensor()};
+  }
+};
+
+// ---- Public attention calls. ---------------------------------------------------------------------------------
+
+void check_shapes(const Tensor& q, const Tensor& k, const Tensor& v, const Params& P, const Table& t) {
+  require(q.dim() == 4, "q must be [B,H,N,HD], got ", shape_str(q.sizes()));
+  const int64_t H = q.size(1), HD = q.size(3), J = t.J;
+  require(k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v must have the same shape");
+  auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
+    if (x.defined() && x.sizes() != c10::IntArrayRef(s))
+      require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
+  };
+  expect(P.pb, {J, H}, "pos_bias");
+  expect(P.se, {J, HD}, "scale_embed");
+  expect(P.sg, {H, J}, "score_gain");
+  expect(P.ig, {H}, "if_gain");
+}
+
+Params float_params(const Tensor& pb, const OptTensor& se, const OptTensor& sg, const OptTensor& ig) {
+  auto f = [](const Tensor& t) { return t.defined() ? t.to(at::kFloat) : t; };
+  return {f(pb), f(undef(se)), f(undef(sg)), f(undef(ig))};
+}
+
+bool kernel_dtype(at::ScalarType dt) { return dt == at::kFloat || dt == at::kBFloat16; }
+
+// (out, lse) with the dtype rules of the public functions.
+std::tuple<Tensor, Tensor> attention(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& pb,
+                                     const OptTensor& se, const OptTensor& sg, const OptTensor& ig,
+                                     const py::object& offsets) {
+  const TablePtr t = make_table(offsets);
+  py::gil_scoped_release nogil;
+  check_shapes(q0, k0, v0, {pb, undef(se), undef(sg), undef(ig)}, *t);
+  const auto orig = q0.scalar_type();
+  const auto dt = kernel_dtype(orig) ? orig : at::kBFloat16;
+  const Params P = float_params(pb, se, sg, ig);
+  const variable_list r = AttentionFunction::apply(q0.to(dt), k0.to(dt), v0.to(dt), P.pb, opt(P.se), opt(P.sg),
+                                                   opt(P.ig), t);
+  return {r[0].to(orig), r[1]};
+}
+
+Tensor attention_qkv(const Tensor& qkv0, int64_t H, const Tensor& pb, const OptTensor& se, const OptTensor& sg,
+                     const OptTensor& ig, const py::object& offsets, const OptTensor& kd, const OptTensor& vd) {
+  const TablePtr t = make_table(offsets);
+  py::gil_scoped_release nogil;
+  const int64_t E3 = qkv0.size(2);
+  require(H > 0 && E3 % (3 * H) == 0, "qkv last dim ", E3, " is not 3 * num_heads * head_dim");
+  const std::vector<int64_t> heads{qkv0.size(0), H, qkv0.size(1), E3 / (3 * H)};
+  auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
+    if (x.defined() && x.sizes() != c10::IntArrayRef(s))
+      require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
+  };
+  expect(pb, {t->J, H}, "pos_bias");
+  expect(undef(se), {t->J, heads[3]}, "scale_embed");
+  expect(undef(sg), {H, t->J}, "score_gain");
+  expect(undef(ig), {H}, "if_gain");
+  const auto orig = qkv0.scalar_type();
+  const Tensor qkv = kernel_dtype(orig) ? qkv0 : qkv0.to(at::kBFloat16);
+  const Params P = float_params(pb, se, sg, ig);
+  variable_list r;
+  if (!kd.has_value()) {
+    r = AttentionQkvFunction::apply(qkv, P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, t);
+  } else {
+    require(kd->sizes() == c10::IntArrayRef(heads) && vd->sizes() == c10::IntArrayRef(heads),
+            "kv_inject deltas must be torch.Size([", heads[0], ", ", heads[1], ", ", heads[2], ", ", heads[3], "])");
+    r = AttentionQkvKvFunction::apply(qkv, *kd, *vd, P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, t);
+  }
+  return r[0].to(orig);
+}
+
+// ---- Decode step. ----------------------------------------------------------------------------------------------
+
+Tensor decode(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& k_ring, const Tensor& v_ring,
+              const Tensor& pos0, const Tensor& pb0, const OptTensor& se0, const OptTensor& sg0,
+              const OptTensor& ig0, const py::object& offsets) {
+  const TablePtr t = make_table(offsets);
+  py::gil_scoped_release nogil;
+  auto f32 = [](const Tensor& x) { return x.defined() ? x.detach().to(at::kFloat).contiguous() : x; };
+  const Tensor q = q0.contiguous(), k = k0.contiguous(), v = v0.contiguous();
+  const Tensor pos = pos0.to(at::kLong).contiguous();
+  const Tensor pb = f32(pb0), se = f32(undef(se0)), sg = f32(undef(sg0)), ig = f32(undef(ig0));
+  const Tensor out = at::empty_like(q);
+  const c10::Device dev = require_gpu({&q, &k, &v, &k_ring, &v_ring, &pos, &pb, &out});
+  const c10::OptionalDeviceGuard guard(dev);
+  require(k_ring.dim() == 4, "k_ring must be [B,H,S,D], got ", shape_str(k_ring.sizes()));
+  const int64_t B = k_ring.size(0), H = k_ring.size(1), S = k_ring.size(2), D = k_ring.size(3);
+  const auto dt = q.scalar_type();
+  require(kernel_dtype(dt) && k.scalar_type() == dt && v.scalar_type() == dt && k_ring.scalar_type() == dt &&
+              v_ring.scalar_type() == dt, "q, k_new, v_new, rings and out must share dtype float32 or bfloat16");
+  auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
+    if (x.sizes() != c10::IntArrayRef(s) || !x.is_contiguous())
+      require(false, name, " must be a contiguous ", shape_str(s), " tensor, got ", shape_str(x.sizes()),
+              " (contiguous=", x.is_contiguous() ? "True" : "False", ")");
+  };
+  expect(q, {B, H, D}, "q");
+  expect(k, {B, H, D}, "k_new");
+  expect(v, {B, H, D}, "v_new");
+  expect(v_ring, {B, H, S, D}, "v_ring");
+  require(k_ring.is_contiguous(), "k_ring must be contiguous");
+  require(pos.dim() == 1 && pos.size(0) == B, "pos must be a contiguous int64 [B] tensor");
+  dsqg_decode_args a = {};
+  fill_shape(a.shape, dt, B, H, 0, D, *t);
+  a.S = (int32_t)S;
+  a.q = ptr(q); a.k_new = ptr(k); a.v_new = ptr(v);
+  a.k_ring = ptr(k_ring); a.v_ring = ptr(v_ring);
+  a.pos = static_cast<const int64_t*>(ptr(pos));
+  a.pos_bias = static_cast<const float*>(ptr(pb));
+  a.scale_embed = static_cast<const float*>(ptr(se));
+  a.score_gain = static_cast<const float*>(ptr(sg));
+  a.if_gain = static_cast<const float*>(ptr(ig));
+  a.out = ptr(out);
+  check(api.decode_step(&a, stream_of(dev)), "dsqg_decode_step");
+  // The rings were written in place.
+  for (const Tensor* r : {&k_ring, &v_ring})
+    if (!r->is_inference()) r->unsafeGetTensorImpl()->bump_version();
+  return out;
+}
+
+// ---- Causal-mean pool with a sigmoid gate. ---------------------------------------------------------------------
+
+int pool_code(at::ScalarType dt) { return dt == at::kFloat ? DSQG_F32 : dt == at::kBFloat16 ? DSQG_BF16 : DSQG_F16; }
+
+Tensor pool_ready(const Tensor& t, const Tensor& like, const char* name) {
+  const int64_t B = like.size(0), N = like.size(1), C = like.size(2);
+  if (t.sizes() != like.sizes())
+    require(false, name, " must be [", B, ",", N, ",", C, "], got ", shape_str(t.sizes()));
+  const auto dt = t.scalar_type();
+  require(dt == at::kFloat || dt == at::kBFloat16 || dt == at::kHalf, name,
+          " must be float32, bfloat16 or float16, got ", dt);
+  return rows_ready(t.numel() && t.stride(1) < C ? t.contiguous() : t);  // overlapping rows: copy
+}
+
+Tensor pool_workspace(const Tensor& x, bool backward) {
+  size_t n = 0;
+  check(api.pool_workspace_size((int32_t)x.size(0), (int32_t)x.size(1), (int32_t)x.size(2), backward, &n),
+        "dsqg_pool_gate_workspace_size");
+  return at::empty({std::max<int64_t>((int64_t)n, 1)}, x.options().dtype(at::kByte));
+}
+
+void set_strides(int64_t (&dst)[2], const Tensor& t) { dst[0] = t.stride(0); dst[1] = t.stride(1); }
+
+struct PoolFunction : torch::autograd::Function<PoolFunction> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x0, const Tensor& g0) {
+    const c10::Device dev = require_gpu({&x0, &g0});
+    const c10::OptionalDeviceGuard guard(dev);
+    const Tensor x = pool_ready(x0, x0, "x"), g = pool_ready(g0, x0, "gate_pre"), ws = pool_workspace(x, false);
+    const Tensor out = at::empty(x.sizes(), x.options().dtype(at::promote_types(x.scalar_type(), g.scalar_type())));
+    dsqg_pool_gate_fwd_args a = {};
+    a.B = (int32_t)x.size(0); a.N = (int32_t)x.size(1); a.C = (int32_t)x.size(2);
+    a.x_dtype = pool_code(x.scalar_type()); a.gate_dtype = pool_code(g.scalar_type());
+    a.out_dtype = pool_code(out.scalar_type());
+    a.x = ptr(x); set_strides(a.x_stride, x);
+    a.gate_pre = ptr(g); set_strides(a.gate_stride, g);
+    a.out = ptr(out); set_strides(a.out_stride, out);
+    a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
+    check(api.pool_fwd(&a, stream_of(dev)), "dsqg_pool_gate_fwd");
+    ctx->save_for_backward({x0, g0});
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const bool need_dx = ctx->needs_input_grad(0), need_dg = ctx->needs_input_grad(1);
+    if (!need_dx && !need_dg) return {Tensor(), Tensor()};
+    const c10::Device dev = require_gpu({&s[0], &s[1], &grads[0]});
+    const c10::OptionalDeviceGuard guard(dev);
+    const Tensor x = pool_ready(s[0], s[0], "x"), g = pool_ready(s[1], s[0], "gate_pre");
+    const Tensor dy = pool_ready(grads[0], s[0], "dout"), ws = pool_workspace(x, true);
+    Tensor dx, dg;
+    dsqg_pool_gate_bwd_args a = {};
+    a.B = (int32_t)x.size(0); a.N = (int32_t)x.size(1); a.C = (int32_t)x.size(2);
+    a.x_dtype = pool_code(x.scalar_type()); a.gate_dtype = pool_code(g.scalar_type());
+    a.dout_dtype = pool_code(dy.scalar_type());
+    a.x = ptr(x); set_strides(a.x_stride, x);
+    a.gate_pre = ptr(g); set_strides(a.gate_stride, g);
+    a.dout = ptr(dy); set_strides(a.dout_stride, dy);
+    if (need_dx) {
+      dx = at::empty(x.sizes(), x.options());
+      a.dx = ptr(dx); set_strides(a.dx_stride, dx);
+    }
+    if (need_dg) {
+      dg = at::empty(x.sizes(), g.options());
+      a.dgate_pre = ptr(dg); set_strides(a.dgate_stride, dg);
+    }
+    a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
+    check(api.pool_bwd(&a, stream_of(dev)), "dsqg_pool_gate_bwd");
+    return {dx, dg};
+  }
+};
+
+Tensor pool_gate(const Tensor& x, const Tensor& g) {
+  py::gil_scoped_release nogil;
+  return PoolFunction::apply(x, g);
+}
+
+void init(const py::dict& addresses, const py::object& library_error) {
+  auto get = [&](auto& fn, const char* name) {
+    fn = reinterpret_cast<std::decay_t<decltype(fn)>>(addresses[name].cast<uintptr_t>());
+  };
+  get(api.status_string, "dsqg_status_string");
+  get(api.fwd, "dsqg_fwd");
+  get(api.bwd_workspace_size, "dsqg_bwd_workspace_size");
+  get(api.bwd, "dsqg_bwd");
+  get(api.decode_step, "dsqg_decode_step");
+  get(api.pool_workspace_size, "dsqg_pool_gate_workspace_size");
+  get(api.pool_fwd, "dsqg_pool_gate_fwd");
+  get(api.pool_bwd, "dsqg_pool_gate_bwd");
+  api.library_error = library_error.inc_ref().ptr();  // lives as long as the process
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_dsqg_host, m) {
+  m.doc() = "Native host layer of dwarf_amd's eager public functions.";
+  m.def("init", &init);
+  m.def("attention", &attention);
+  m.def("attention_qkv", &attention_qkv);
+  m.def("decode", &decode);
+  m.def("pool_gate", &pool_gate);
+}

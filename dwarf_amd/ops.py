@@ -5,6 +5,8 @@ The ops take device tensors, pass raw pointers, element strides and the current 
 to libdsqg_hip.so through ctypes, and allocate their outputs (and the backward workspace) with
 torch's caching allocator.  ``dwarf::dsqg_fwd`` carries an autograd formula that calls
 ``dwarf::dsqg_bwd``, and every op has a fake (meta) implementation so graphs can be traced.
+They are what traced code sees; the eager public functions (api.py) call the same library through
+the native host layer.
 
 Tensors must live on a ROCm GPU: there is no CPU path, and a missing library raises.
 
@@ -19,6 +21,7 @@ from typing import List, Optional, Tuple
 
 import torch
 from torch import Tensor
+from torch._subclasses.fake_tensor import FakeTensor
 
 from . import _lib
 from .offsets import long_range_taps
@@ -271,7 +274,7 @@ def _setup_context(ctx, inputs, output):
     ctx.mark_non_differentiable(lse, alpha_lr)
 
 
-def _backward(ctx, dout, _dlse, _dalpha, direct: bool = False):
+def _backward(ctx, dout, _dlse, _dalpha):
     q, k, v, lse, alpha_lr, pos_bias, scale_embed, score_gain, if_gain = ctx.saved_tensors
     need = ctx.needs_input_grad
     need_dse = bool(need[4]) and scale_embed is not None
@@ -279,12 +282,7 @@ def _backward(ctx, dout, _dlse, _dalpha, direct: bool = False):
     need_da = bool(need[6]) and if_gain is not None
     args = (q, k, v, dout.to(q.dtype), lse, alpha_lr, pos_bias, scale_embed, score_gain, if_gain,
             ctx.offsets, need_dse, need_dg, need_da)
-    if direct:
-        launch = BwdLaunch(*args[:5], *args[6:], alpha_lr=alpha_lr)
-        launch.run()
-        dq, dk, dv, dpb, dse, dg, da = launch.outputs()
-    else:
-        dq, dk, dv, dpb, dse, dg, da = dsqg_bwd(*args)
+    dq, dk, dv, dpb, dse, dg, da = dsqg_bwd(*args)
     return (dq, dk, dv, dpb.to(pos_bias.dtype),
             dse.to(scale_embed.dtype) if need_dse else None,
             dg.to(score_gain.dtype) if need_dg else None,
@@ -303,7 +301,7 @@ def _setup_context_qkv(ctx, inputs, output):
     ctx.mark_non_differentiable(lse, alpha_lr)
 
 
-def _backward_qkv(ctx, dout, _dlse, _dalpha, direct: bool = False):
+def _backward_qkv(ctx, dout, _dlse, _dalpha):
     qkv, lse, alpha_lr, pos_bias, scale_embed, score_gain, if_gain = ctx.saved_tensors
     need = ctx.needs_input_grad
     need_dse = bool(need[3]) and scale_embed is not None
@@ -311,8 +309,7 @@ def _backward_qkv(ctx, dout, _dlse, _dalpha, direct: bool = False):
     need_da = bool(need[5]) and if_gain is not None
     args = (qkv, ctx.num_heads, dout.to(qkv.dtype), lse, alpha_lr, pos_bias, scale_embed,
             score_gain, if_gain, ctx.offsets, need_dse, need_dg, need_da)
-    bwd = _bwd_qkv_impl if direct else dsqg_bwd_qkv
-    dqkv, dpb, dse, dg, da = bwd(*args)
+    dqkv, dpb, dse, dg, da = dsqg_bwd_qkv(*args)
     return (dqkv, None, dpb.to(pos_bias.dtype),
             dse.to(scale_embed.dtype) if need_dse else None,
             dg.to(score_gain.dtype) if need_dg else None,
@@ -430,7 +427,7 @@ def _setup_context_qkv_kv(ctx, inputs, output):
     ctx.mark_non_differentiable(lse, alpha_lr, k_eff, v_eff)
 
 
-def _backward_qkv_kv(ctx, dout, _dlse, _dalpha, _dk_eff, _dv_eff, direct: bool = False):
+def _backward_qkv_kv(ctx, dout, _dlse, _dalpha, _dk_eff, _dv_eff):
     qkv, k_eff, v_eff, lse, alpha_lr, pos_bias, scale_embed, score_gain, if_gain = ctx.saved_tensors
     need = ctx.needs_input_grad
     need_dse = bool(need[5]) and scale_embed is not None
@@ -438,12 +435,7 @@ def _backward_qkv_kv(ctx, dout, _dlse, _dalpha, _dk_eff, _dv_eff, direct: bool =
     need_da = bool(need[7]) and if_gain is not None
     args = (qkv, k_eff, v_eff, ctx.num_heads, dout.to(qkv.dtype), lse, alpha_lr, pos_bias,
             scale_embed, score_gain, if_gain, ctx.offsets, need_dse, need_dg, need_da)
-    if direct:
-        dqkv, dpb, dse, dg, da = _bwd_qkv_impl(
-            qkv, ctx.num_heads, dout.to(qkv.dtype), lse, alpha_lr, pos_bias, scale_embed,
-            score_gain, if_gain, ctx.offsets, need_dse, need_dg, need_da, k_eff, v_eff)
-    else:
-        dqkv, dpb, dse, dg, da = dsqg_bwd_qkv_kv(*args)
+    dqkv, dpb, dse, dg, da = dsqg_bwd_qkv_kv(*args)
     _, dk, dv = split_qkv(dqkv, ctx.num_heads)
     return (dqkv, dk.to(ctx.delta_dtypes[0]), dv.to(ctx.delta_dtypes[1]), None,
             dpb.to(pos_bias.dtype),
@@ -456,67 +448,14 @@ torch.library.register_autograd("dwarf::dsqg_fwd_qkv_kv", _backward_qkv_kv,
                                 setup_context=_setup_context_qkv_kv)
 
 
-# Eager autograd over the same launch objects: the custom ops above are what traced code
-# (torch.compile, export, fake tensors) sees; outside tracing the public functions take these
-# Functions, which skip the custom-op dispatch (about 100 us of host time per forward +
-# backward, measured on the MI355X host, where the kernels themselves take a few tens of us
-# at small shapes).  Same kernels, same results.
-
 def traced(*tensors) -> bool:
-    """True under torch.compile / export or for fake or meta tensors: use the custom ops."""
-    if torch.compiler.is_compiling():
+    """True where the public functions must go through the custom ops: under torch.compile /
+    export, a dispatch mode (make_fx, fake tensors) or jit tracing, and for fake or meta tensors.
+    Eager code takes the native host layer (csrc/dsqg_host.cpp): same kernels, same results."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
+            or torch._C._get_tracing_state() is not None:
         return True
-    from torch._subclasses.fake_tensor import FakeTensor
-    return any(isinstance(t, FakeTensor) or (t is not None and t.device.type == "meta")
-               for t in tensors)
-
-
-class AttentionFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, pos_bias, scale_embed, score_gain, if_gain, offsets):
-        launch = FwdLaunch(q, k, v, pos_bias, scale_embed, score_gain, if_gain, offsets)
-        launch.run()
-        outs = (launch.out, launch.lse, launch.alpha_lr)
-        _setup_context(ctx, (q, k, v, pos_bias, scale_embed, score_gain, if_gain, offsets), outs)
-        return outs
-
-    @staticmethod
-    def backward(ctx, dout, dlse, dalpha):
-        return _backward(ctx, dout, dlse, dalpha, direct=True)
-
-
-class AttentionQkvFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, qkv, num_heads, pos_bias, scale_embed, score_gain, if_gain, offsets):
-        q, k, v = split_qkv(qkv, num_heads)
-        launch = FwdLaunch(q, k, v, pos_bias, scale_embed, score_gain, if_gain, offsets)
-        launch.run()
-        outs = (launch.out, launch.lse, launch.alpha_lr)
-        _setup_context_qkv(ctx, (qkv, num_heads, pos_bias, scale_embed, score_gain, if_gain,
-                                 offsets), outs)
-        return outs
-
-    @staticmethod
-    def backward(ctx, dout, dlse, dalpha):
-        return _backward_qkv(ctx, dout, dlse, dalpha, direct=True)
-
-
-class AttentionQkvKvFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, qkv, k_delta, v_delta, num_heads, pos_bias, scale_embed, score_gain, if_gain,
-                offsets):
-        k_eff, v_eff = _kv_eff(qkv, k_delta, v_delta, num_heads)
-        q = split_qkv(qkv, num_heads)[0]
-        launch = FwdLaunch(q, k_eff, v_eff, pos_bias, scale_embed, score_gain, if_gain, offsets)
-        launch.run()
-        outs = (launch.out, launch.lse, launch.alpha_lr, k_eff, v_eff)
-        _setup_context_qkv_kv(ctx, (qkv, k_delta, v_delta, num_heads, pos_bias, scale_embed,
-                                    score_gain, if_gain, offsets), outs)
-        return outs
-
-    @staticmethod
-    def backward(ctx, dout, dlse, dalpha, dk_eff, dv_eff):
-        return _backward_qkv_kv(ctx, dout, dlse, dalpha, dk_eff, dv_eff, direct=True)
+    return any(isinstance(t, FakeTensor) or t.device.type == "meta" for t in tensors)
 
 
 # ------------------------------------------------------------------------------------------
@@ -708,23 +647,3 @@ def _pool_backward(ctx, dout):
 torch.library.register_autograd("dwarf::pool_gate_fwd", _pool_backward,
                                 setup_context=_pool_setup_context)
 
-
-class PoolGateFn(torch.autograd.Function):
-    """Eager autograd of the pool over the launch objects (see AttentionFn)."""
-
-    @staticmethod
-    def forward(ctx, x, gate_pre):
-        launch = PoolLaunch(x, gate_pre)
-        launch.run()
-        ctx.save_for_backward(x, gate_pre)
-        return launch.out
-
-    @staticmethod
-    def backward(ctx, dout):
-        x, gate_pre = ctx.saved_tensors
-        need_dx, need_dg = bool(ctx.needs_input_grad[0]), bool(ctx.needs_input_grad[1])
-        if not (need_dx or need_dg):
-            return None, None
-        launch = PoolLaunch(x, gate_pre, dout, need_dx, need_dg)
-        launch.run()
-        return (launch.dx if need_dx else None), (launch.dgate if need_dg else None)
