@@ -88,7 +88,7 @@ BwdLayout bwd_layout(const dsqg_bwd_args& a, const BwdParams& p) {
   return L;
 }
 
-int check_bwd(const dsqg_bwd_args* a, BwdParams* p) {
+int check_bwd(const dsqg_bwd_args* a, BwdParams* p, bool compact = false) {
   if (!a) return DSQG_EINVAL;
   const dsqg_shape& s = a->shape;
   memset(p, 0, sizeof(*p));
@@ -112,7 +112,7 @@ int check_bwd(const dsqg_bwd_args* a, BwdParams* p) {
   p->B = s.B; p->H = s.H; p->N = s.N;
   p->qs = to_strides(a->q_stride); p->ks = to_strides(a->k_stride);
   p->vs = to_strides(a->v_stride); p->dos = to_strides(a->dout_stride);
-  bwd_plan(*p, s.D, s.dtype, a->scale_embed != nullptr || a->dscale_embed != nullptr);
+  bwd_plan(*p, s.D, s.dtype, a->scale_embed != nullptr || a->dscale_embed != nullptr, compact);
   if (s.dtype == DSQG_BF16 && !bwd_mfma_supported(*p, s.D, s.dtype)) return DSQG_EUNSUPPORTED;
   if ((long long)s.B * s.H * p->n_chunks > INT_MAX / 2) return DSQG_EINVAL;  // >= the partial count
   if ((long long)s.B * s.H * p->n_tiles_kv > INT_MAX / 2) return DSQG_EINVAL;
@@ -226,9 +226,14 @@ static int run_bwd(const dsqg_bwd_args* a, int phases, dsqg_stream_t stream, boo
   int st = check_bwd(a, &p);
   if (st) return st;
   const dsqg_shape& s = a->shape;
-  const BwdLayout L = bwd_layout(*a, p);
+  BwdLayout L = bwd_layout(*a, p);
   char* ws = static_cast<char*>(a->workspace);
   if (use_scratch) {
+    // A plan that does not fit gives way to the one with the smallest workspace.
+    if (L.total > DSQG_NOALLOC_SCRATCH_BYTES) {
+      if ((st = check_bwd(a, &p, true))) return st;
+      L = bwd_layout(*a, p);
+    }
     // Sizes are checked before any HIP call; the scratch pointer of this stream's device is
     // taken (once per device) only for a call that fits.
     if (L.total > DSQG_NOALLOC_SCRATCH_BYTES) return DSQG_ETOOLARGE;

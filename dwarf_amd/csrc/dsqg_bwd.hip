@@ -51,7 +51,30 @@ bool bwd_f32_supported(const BwdParams& p, int D, int dtype) {
   return dtype == 0 && f32_mfma_strides_ok(p.N, p.taps.maxd, D, rs, 4);
 }
 
-void bwd_plan(BwdParams& p, int D, int dtype, bool se) {
+// Batches a workgroup of the bf16 scale_embed dq takes (bwd_plan): the choice of 1, 2 and 4 whose
+// rounds of resident workgroups times batches cost least, counting a partial's store and re-read
+// as 0.6 of a tile (fitted to both directions below).  Whole backward, us, at 1 / 2 / 4 batches:
+//   B4 H4 N256 D64     27.8 / 37.1 / 56.6      B4 H8 N2047 D80     76 /  70 /  84
+//   B8 H8 N512 D32     28.2 / 33.4 / 45.6      B16 H8 N2048 D32   118 / 107 / 113
+//   B4 H8 N1024 D64    39.3 / 46.5 / 62.7      B8 H6 N2048 D128   233 / 215 / 237
+//   B2 H12 N2048 D64   46.8 / 51.5             B8 H12 N2048 D64   144 / 134 / 133
+//   B8 H8 N2048 D96     151 /  139 /  139      B8 H16 N2048 D96   303 / 272 / 261
+static int se_batches(const BwdParams& p, int D) {
+  const int ns = p.taps.J - p.taps.W - 1;
+  const int slots = 256 * (D == 128 ? 1 : (D > 64 || ns != 11 ? 2 : 3));  // resident workgroups
+  int best = 1;
+  double best_cost = 0;
+  for (int n : {1, 2, 4}) {
+    if (n > 1 && n / 2 >= p.B) break;
+    const int nb = n < p.B ? n : (p.B > 0 ? p.B : 1);
+    const long long wgs = (long long)((p.B + nb - 1) / nb) * p.H * p.n_tiles;
+    const double cost = (double)nb * ((wgs + slots - 1) / slots) + 0.6 * wgs / slots;
+    if (n == 1 || cost < best_cost) { best = nb; best_cost = cost; }
+  }
+  return best;
+}
+
+void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool compact) {
   const bool mfma = bwd_mfma_supported(p, D, dtype);
   const bool tile64 = mfma || bwd_f32_supported(p, D, dtype);
   const int QPB = tile64 ? 64 : kBlock / lanes_per_row(D);  // dq rows per tile
@@ -60,15 +83,16 @@ void bwd_plan(BwdParams& p, int D, int dtype, bool se) {
   p.n_tiles_kv = (p.N + KPB - 1) / KPB;
   // One tile per workgroup: the partial rows (J floats) are small next to a tile's loads, and the
   // single-tile form keeps no per-lane addresses across tiles.  The bf16 dq with scale_embed
-  // takes the same head and tile of four batches per workgroup instead: its [J x D] fp32 dse
+  // takes the same head and tile of up to four batches per workgroup instead: its [J x D] fp32 dse
   // partial is as large as a tile's dS, so one per tile costs as many bytes again as the tile's
-  // dq (written, then read back by the reduction); one per four tiles cuts them to a quarter.
+  // dq (written, then read back by the reduction); one per four tiles cuts them to a quarter, where
+  // the grid still fills the chip (se_batches; compact: four, the smallest workspace).
   // (Four consecutive tiles of one (b,h) instead put every tile of four times as many (b,h)
   // slices in flight at once, which overflowed L2: 143 MB more L2-miss reads per launch.)
   // dse sums over every b and h, dbias / dg / da over b, so a partial may span batches.
   p.tiles_per_block = 1;
   p.n_chunks = p.n_tiles;
-  p.batches_per_block = (mfma && se) ? (p.B < 4 ? (p.B > 0 ? p.B : 1) : 4) : 1;
+  p.batches_per_block = !(mfma && se) ? 1 : compact ? (p.B < 4 ? (p.B > 0 ? p.B : 1) : 4) : se_batches(p, D);
   p.n_bgroups = (p.B + p.batches_per_block - 1) / p.batches_per_block;
 }
 

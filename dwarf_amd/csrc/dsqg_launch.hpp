@@ -24,8 +24,9 @@ hipError_t launch_bwd_dq_f32(const BwdParams& p, int D, unsigned nblocks, hipStr
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
 
 // Tiling of the backward for these sizes and kernel choice; fills n_tiles / tiles_per_block /
-// n_chunks / n_tiles_kv (se: scale_embed or its gradient is present).
-void bwd_plan(BwdParams& p, int D, int dtype, bool se);
+// n_chunks / n_tiles_kv (se: scale_embed or its gradient is present; compact: the plan with the
+// smallest workspace instead of the fastest).
+void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool compact);
 
 // bf16 MFMA backward kernels: same conditions as the MFMA forward.
 bool bwd_mfma_supported(const BwdParams& p, int D, int dtype);

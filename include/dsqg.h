@@ -204,7 +204,9 @@ int dsqg_bwd_params(const dsqg_bwd_args* args, dsqg_stream_t stream);
  * called.  Its address is looked up once per device on the first call there (hipGetSymbolAddress):
  * make that first call outside stream capture (one eager call), later calls may be captured
  * into a HIP graph (the call issues kernel launches only, no memset and no allocation).  A call whose
- * workspace (dsqg_bwd_workspace_size) exceeds it returns DSQG_ETOOLARGE before any HIP call.
+ * workspace (dsqg_bwd_workspace_size) exceeds it takes the launch plan with the smallest workspace
+ * instead (dscale_embed partials over four batches each), and if that does not fit either returns
+ * DSQG_ETOOLARGE before any HIP call.
  * Same kernels, outputs and stream rules as dsqg_bwd; calls that overlap on one device (other
  * streams, other threads) share the scratch and race, so serialise them. */
 int dsqg_bwd_noalloc(const dsqg_bwd_args* args, dsqg_stream_t stream);
