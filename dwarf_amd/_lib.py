@@ -93,6 +93,13 @@ class PoolBwdArgs(ctypes.Structure):
                 ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t)]
 
 
+class LinearWgradArgs(ctypes.Structure):
+    _fields_ = [("T", ctypes.c_int32), ("O", ctypes.c_int32), ("I", ctypes.c_int32),
+                ("dtype", ctypes.c_int32), ("dy", _vp), ("dy_stride", ctypes.c_int64),
+                ("x", _vp), ("x_stride", ctypes.c_int64), ("dw", _vp), ("db", _vp),
+                ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t)]
+
+
 # Every symbol include/dsqg.h declares, with its ctypes signature.
 SIGNATURES = {
     "dsqg_abi_version": (ctypes.c_int, []),
@@ -114,6 +121,9 @@ SIGNATURES = {
                                                      ctypes.POINTER(ctypes.c_size_t)]),
     "dsqg_pool_gate_fwd": (ctypes.c_int, [ctypes.POINTER(PoolFwdArgs), _vp]),
     "dsqg_pool_gate_bwd": (ctypes.c_int, [ctypes.POINTER(PoolBwdArgs), _vp]),
+    "dsqg_linear_wgrad_workspace_size": (ctypes.c_int, [ctypes.POINTER(LinearWgradArgs),
+                                                        ctypes.POINTER(ctypes.c_size_t)]),
+    "dsqg_linear_wgrad": (ctypes.c_int, [ctypes.POINTER(LinearWgradArgs), _vp]),
 }
 
 _LIB = None

@@ -9,6 +9,7 @@
 //
 // The entry points of libdsqg_hip.so arrive as addresses from the loader (dwarf_amd/_lib.py), so
 // the library that was checked there is the one called here.  Nothing is kept between calls.
+#include <ATen/autocast_mode.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
@@ -35,6 +36,8 @@ struct Api {
   decltype(&dsqg_pool_gate_workspace_size) pool_workspace_size = nullptr;
   decltype(&dsqg_pool_gate_fwd) pool_fwd = nullptr;
   decltype(&dsqg_pool_gate_bwd) pool_bwd = nullptr;
+  decltype(&dsqg_linear_wgrad_workspace_size) linear_workspace_size = nullptr;
+  decltype(&dsqg_linear_wgrad) linear_wgrad = nullptr;
   PyObject* library_error = nullptr;  // dwarf_amd._lib.DSQGLibraryError
 } api;
 
@@ -536,6 +539,98 @@ Tensor pool_gate(const Tensor& x, const Tensor& g) {
   return PoolFunction::apply(x, g);
 }
 
+// ---- Linear layers: the library's products, and dW and db from one kernel pair. -----------------------------------
+
+// Whether the weight gradient goes to dsqg_linear_wgrad: 16-bit operands of aligned widths, and an
+// output small enough that the library's tiling of it alone leaves most of the chip idle.  Against
+// its product and column sum (us, 16-bit, rows x O x I): 512 x 256 x 256 12 / 40,
+// 16384 x 256 x 256 17 / 122, 16384 x 768 x 768 50 / 124, 16384 x 3072 x 768 157 / 224,
+// 65536 x 2304 x 768 430 / 609; 65536 x 3072 x 768 578 / 548.
+bool use_wgrad(at::ScalarType dt, int64_t T, int64_t O, int64_t I) {
+  if ((dt != at::kHalf && dt != at::kBFloat16) || T < 1 || O % 8 != 0 || I % 8 != 0) return false;
+  if ((T + 128) * std::max(O, I) * 2 >= (1ll << 31)) return false;
+  return O * I <= (1ll << 21) || (O * I <= 3072 * 768 && T <= 16384);
+}
+
+// [T, C] rows the kernel reads in place (unit column stride, 16-byte aligned rows that do not
+// overlap), else a copy.
+Tensor wgrad_rows(const Tensor& t) {
+  const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 &&
+                  (t.size(0) + 128) * t.stride(0) * 2 < (1ll << 31) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
+void linear_wgrad(const Tensor& dy0, const Tensor& x0, bool need_db, Tensor& dw, Tensor& db) {
+  const c10::Device dev = require_gpu({&dy0, &x0});
+  const c10::OptionalDeviceGuard guard(dev);
+  const Tensor dy = wgrad_rows(dy0), x = wgrad_rows(x0);
+  dw = at::empty({dy.size(1), x.size(1)}, x.options());
+  if (need_db) db = at::empty({dy.size(1)}, x.options());
+  dsqg_linear_wgrad_args a = {};
+  a.T = (int32_t)dy.size(0); a.O = (int32_t)dy.size(1); a.I = (int32_t)x.size(1);
+  a.dtype = pool_code(x.scalar_type());
+  a.dy = dy.data_ptr(); a.dy_stride = dy.stride(0);
+  a.x = x.data_ptr(); a.x_stride = x.stride(0);
+  a.dw = dw.data_ptr();
+  a.db = need_db ? db.data_ptr() : nullptr;
+  size_t nbytes = 0;
+  check(api.linear_workspace_size(&a, &nbytes), "dsqg_linear_wgrad_workspace_size");
+  const Tensor ws = at::empty({(int64_t)nbytes}, x.options().dtype(at::kByte));
+  a.workspace = ws.data_ptr(); a.workspace_bytes = nbytes;
+  check(api.linear_wgrad(&a, stream_of(dev)), "dsqg_linear_wgrad");
+}
+
+struct LinearFunction : torch::autograd::Function<LinearFunction> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& b) {
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["bias"] = b.has_value();
+    return at::linear(x, w, b);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    const variable_list s = ctx->get_saved_variables();
+    const Needs n(ctx, {true, true, ctx->saved_data["bias"].toBool()});
+    const Tensor &x = s[0], &w = s[1], &dy = g[0];
+    const int64_t O = w.size(0), I = w.size(1);
+    Tensor dx, dw, db;
+    if (n.need[0]) dx = at::matmul(dy, w);
+    if (n.need[1] || n.need[2]) {
+      const Tensor dy2 = dy.reshape({-1, O});
+      // Under create_graph the gradients are themselves differentiated: plain products.
+      if (n.need[1] && !at::GradMode::is_enabled() && dy.scalar_type() == x.scalar_type() &&
+          use_wgrad(x.scalar_type(), dy2.size(0), O, I)) {
+        linear_wgrad(dy2, x.reshape({-1, I}), n.need[2], dw, db);
+      } else {
+        if (n.need[1]) dw = dy2.t().mm(x.reshape({-1, I}));
+        if (n.need[2]) db = dy2.sum(0);
+      }
+    }
+    return {dx, dw, db};
+  }
+};
+
+// F.linear on GPU tensors.  Under autocast the operands are cast as F.linear's are (the same cached
+// weight casts); anything but 16-bit training on plain tensors is F.linear itself.
+Tensor linear(const Tensor& x0, const Tensor& w0, const OptTensor& b0) {
+  py::gil_scoped_release nogil;
+  auto plain = [](const Tensor& t) { return t.is_cuda() && !t.key_set().has(c10::DispatchKey::Python); };
+  if (!at::GradMode::is_enabled() || !w0.requires_grad() || !plain(x0) || !plain(w0) || (b0 && !plain(*b0)) ||
+      x0.dim() < 2 || w0.dim() != 2 || x0.numel() == 0)
+    return at::linear(x0, w0, b0);
+  Tensor x = x0, w = w0;
+  OptTensor b = b0;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) {
+    const auto dt = at::autocast::get_autocast_dtype(at::kCUDA);
+    x = at::autocast::cached_cast(dt, x, at::kCUDA);
+    w = at::autocast::cached_cast(dt, w, at::kCUDA);
+    if (b) b = at::autocast::cached_cast(dt, *b, at::kCUDA);
+  }
+  const auto dt = x.scalar_type();
+  if (dt != w.scalar_type() || (b && dt != b->scalar_type()) || x.size(-1) != w.size(1) ||
+      !use_wgrad(dt, x.numel() / x.size(-1), w.size(0), w.size(1)))
+    return at::linear(x0, w0, b0);
+  return LinearFunction::apply(x, w, b);
+}
+
 void init(const py::dict& addresses, const py::object& library_error) {
   auto get = [&](auto& fn, const char* name) {
     fn = reinterpret_cast<std::decay_t<decltype(fn)>>(addresses[name].cast<uintptr_t>());
@@ -548,6 +643,8 @@ void init(const py::dict& addresses, const py::object& library_error) {
   get(api.pool_workspace_size, "dsqg_pool_gate_workspace_size");
   get(api.pool_fwd, "dsqg_pool_gate_fwd");
   get(api.pool_bwd, "dsqg_pool_gate_bwd");
+  get(api.linear_workspace_size, "dsqg_linear_wgrad_workspace_size");
+  get(api.linear_wgrad, "dsqg_linear_wgrad");
   api.library_error = library_error.inc_ref().ptr();  // lives as long as the process
 }
 
@@ -560,4 +657,5 @@ PYBIND11_MODULE(_dsqg_host, m) {
   m.def("attention_qkv", &attention_qkv);
   m.def("decode", &decode);
   m.def("pool_gate", &pool_gate);
+  m.def("linear", &linear);
 }

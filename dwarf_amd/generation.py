@@ -26,7 +26,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from .modules import FFN, DSQGBlock
+from .modules import FFN, DSQGBlock, Linear
 
 
 class FullCausalAttention(nn.Module):
@@ -39,9 +39,9 @@ class FullCausalAttention(nn.Module):
         self.embedding_dim = embedding_dim
         self.num_heads = num_heads
         self.head_dim = embedding_dim // num_heads
-        self.qkv_proj = nn.Linear(embedding_dim, 3 * embedding_dim, bias=True)
-        self.out_proj = nn.Linear(embedding_dim, embedding_dim, bias=True)
-        self.gate_proj = nn.Linear(embedding_dim, embedding_dim, bias=True)
+        self.qkv_proj = Linear(embedding_dim, 3 * embedding_dim, bias=True)
+        self.out_proj = Linear(embedding_dim, embedding_dim, bias=True)
+        self.gate_proj = Linear(embedding_dim, embedding_dim, bias=True)
         nn.init.constant_(self.gate_proj.bias, 0.0)
         self.dropout_p = dropout
 

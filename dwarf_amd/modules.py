@@ -35,12 +35,27 @@ import math
 from typing import Optional, Sequence, Tuple
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.overrides import has_torch_function
 
-from . import ops
+from . import _lib, ops
 from .api import DSQGRingCache, causal_mean_pool_gate, dsqg_attention_qkv
 from .offsets import OFFSETS_V3, validate
+
+
+class Linear(nn.Linear):
+    """nn.Linear whose weight and bias gradients, in 16-bit training on the GPU, come from one
+    split-row kernel pair (csrc/dsqg_linear.hip) instead of a product tiled over the small weight
+    alone and a column sum.  Parameters, hooks, autocast and results' types are nn.Linear's."""
+
+    def forward(self, x: Tensor) -> Tensor:
+        if not x.is_cuda or ops.traced(x, self.weight) or fwAD._current_level >= 0 \
+                or has_torch_function((x, self.weight)) \
+                or torch._C._functorch.peek_interpreter_stack() is not None:
+            return F.linear(x, self.weight, self.bias)
+        return _lib.host().linear(x, self.weight, self.bias)
 
 
 def _log_linear_bias(offsets: Sequence[int], num_heads: int) -> Tensor:
@@ -65,9 +80,9 @@ class _DSQGBase(nn.Module):
         self.num_heads = num_heads
         self.head_dim = embedding_dim // num_heads
         self._offsets = list(offsets)
-        self.qkv_proj = nn.Linear(embedding_dim, 3 * embedding_dim, bias=True)
-        self.out_proj = nn.Linear(embedding_dim, embedding_dim, bias=True)
-        self.gate_proj = nn.Linear(embedding_dim, embedding_dim, bias=True)
+        self.qkv_proj = Linear(embedding_dim, 3 * embedding_dim, bias=True)
+        self.out_proj = Linear(embedding_dim, embedding_dim, bias=True)
+        self.gate_proj = Linear(embedding_dim, embedding_dim, bias=True)
         nn.init.constant_(self.gate_proj.bias, gate_bias)
         self.pos_bias = nn.Parameter(_log_linear_bias(self._offsets, num_heads))
         self.dropout = nn.Dropout(dropout)
@@ -211,8 +226,8 @@ class FFN(nn.Module):
 
     def __init__(self, embedding_dim: int, ffn_dim: int, dropout: float = 0.1):
         super().__init__()
-        self.fc1 = nn.Linear(embedding_dim, ffn_dim)
-        self.fc2 = nn.Linear(ffn_dim, embedding_dim)
+        self.fc1 = Linear(embedding_dim, ffn_dim)
+        self.fc2 = Linear(ffn_dim, embedding_dim)
         self.drop = nn.Dropout(dropout)
 
     def forward(self, x: Tensor) -> Tensor:
@@ -252,9 +267,9 @@ class DSQGBlock(nn.Module):
         self.ffn = FFN(embedding_dim, ffn_dim, dropout)
         if interference:
             self.inter_norm = nn.LayerNorm(embedding_dim)
-            self.inter_gate = nn.Linear(embedding_dim, embedding_dim)
-            self.inter_k_proj = nn.Linear(embedding_dim, embedding_dim)
-            self.inter_v_proj = nn.Linear(embedding_dim, embedding_dim)
+            self.inter_gate = Linear(embedding_dim, embedding_dim)
+            self.inter_k_proj = Linear(embedding_dim, embedding_dim)
+            self.inter_v_proj = Linear(embedding_dim, embedding_dim)
 
     def _inject(self, inter: Tensor):
         """K/V deltas [B,H,N,HD] (views; the kernels take strides) from inter [B,N,E]."""

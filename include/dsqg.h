@@ -259,6 +259,26 @@ int dsqg_pool_gate_workspace_size(int32_t B, int32_t N, int32_t C, int backward,
 int dsqg_pool_gate_fwd(const dsqg_pool_gate_fwd_args* args, dsqg_stream_t stream);
 int dsqg_pool_gate_bwd(const dsqg_pool_gate_bwd_args* args, dsqg_stream_t stream);
 
+/* Weight and bias gradients of a linear layer y = x W^T + b (the layers around the attention,
+ * train/train_2048_condU.py:126-130, 244-246): dw[o,i] = sum_t dy[t,o] x[t,i] and, when db is
+ * given, db[o] = sum_t dy[t,o].  dy [T,O] and x [T,I] have unit column stride, row strides that are
+ * a multiple of 8 elements and 16-byte aligned bases; O and I are multiples of 8, T >= 1; dw [O,I]
+ * and db [O] are contiguous and 16-byte aligned.  dtype is F16 or BF16, of all four; sums are
+ * fp32 and deterministic, rounded once. */
+typedef struct {
+    int32_t T, O, I;
+    int32_t dtype;             /* DSQG_F16 or DSQG_BF16 */
+    const void* dy;  int64_t dy_stride;
+    const void* x;   int64_t x_stride;
+    void* dw;
+    void* db;                  /* or NULL */
+    void* workspace;           /* 256-byte aligned */
+    size_t workspace_bytes;
+} dsqg_linear_wgrad_args;
+
+int dsqg_linear_wgrad_workspace_size(const dsqg_linear_wgrad_args* args, size_t* bytes);
+int dsqg_linear_wgrad(const dsqg_linear_wgrad_args* args, dsqg_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,136 @@
+"""Weight and bias gradients of the linear layers: the kernel against float64 at the edges of its
+tiles and row splits, and the layer against nn.Linear through autograd and autocast.
+
+A sum of T products rounded once to the 16-bit type is within half an ulp (2^-11 of the value in
+float16, 2^-8 in bfloat16) plus the float32 sum's rounding, below T 2^-24 of its terms' magnitude.
+"""
+
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+from torch import nn
+
+from dwarf_amd import _lib
+from dwarf_amd.modules import Linear
+
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _close(got, dy, x, name):
+    dy, x = dy.double(), x.double()
+    ref, mag = (dy.sum(0), dy.abs().sum(0)) if x.numel() == 0 else (dy.t() @ x, dy.abs().t() @ x.abs())
+    bound = HALF_ULP[got.dtype] * ref.abs() + len(dy) * 2.0 ** -24 * mag + 2.0 ** -25
+    assert ((got.double() - ref).abs() <= bound).all(), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,O,I,pad", [
+    (1, 8, 8, 0), (63, 8, 136, 8), (64, 128, 128, 0), (65, 136, 120, 0), (256, 256, 128, 24),
+    (257, 128, 264, 0), (1000, 264, 520, 0), (8191, 256, 256, 0), (70001, 8, 8, 0)])
+def test_kernel_against_float64(gpu_device, T, O, I, pad, dtype):
+    g = torch.Generator().manual_seed(T + O + I)
+    dy = torch.randn(T, O + pad, generator=g).to(gpu_device, dtype)[:, :O]
+    x = torch.randn(T, I + pad, generator=g).to(gpu_device, dtype)[:, :I]
+    a = _lib.LinearWgradArgs()
+    a.T, a.O, a.I = T, O, I
+    a.dtype = _lib.DSQG_F16 if dtype == torch.float16 else _lib.DSQG_BF16
+    a.dy, a.dy_stride, a.x, a.x_stride = dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0)
+    dw = torch.full((O, I), float("nan"), device=gpu_device, dtype=dtype)
+    db = torch.full((O,), float("nan"), device=gpu_device, dtype=dtype)
+    a.dw, a.db = dw.data_ptr(), db.data_ptr()
+    n = ctypes.c_size_t(0)
+    lib = _lib.load()
+    _lib.check(lib.dsqg_linear_wgrad_workspace_size(ctypes.byref(a), ctypes.byref(n)), "size")
+    ws = torch.empty(n.value, dtype=torch.uint8, device=gpu_device)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n.value
+    stream = torch.cuda.current_stream(gpu_device).cuda_stream
+    _lib.check(lib.dsqg_linear_wgrad(ctypes.byref(a), stream), "dsqg_linear_wgrad")
+    torch.cuda.synchronize(gpu_device)
+    _close(dw, dy, x, "dw")
+    _close(db, dy, x[:, :0], "db")
+
+
+def test_arguments_are_checked_on_the_host():
+    lib = _lib.load()
+    n = ctypes.c_size_t(0)
+    a = _lib.LinearWgradArgs()
+    a.T, a.O, a.I, a.dtype = 64, 16, 24, _lib.DSQG_BF16
+    assert lib.dsqg_linear_wgrad_workspace_size(ctypes.byref(a), ctypes.byref(n)) == _lib.DSQG_OK
+    assert lib.dsqg_linear_wgrad(ctypes.byref(a), None) == _lib.DSQG_EINVAL  # no tensors
+    a.dy = a.x = a.dw = a.db = 0x10000
+    a.dy_stride, a.x_stride = 16, 24
+    assert lib.dsqg_linear_wgrad(ctypes.byref(a), None) == _lib.DSQG_EWORKSPACE
+    for field, value in (("O", 12), ("I", 0), ("T", -1), ("dtype", _lib.DSQG_F32), ("dy_stride", 8),
+                         ("x_stride", 28), ("x", 0x10008)):
+        b = _lib.LinearWgradArgs.from_buffer_copy(a)
+        setattr(b, field, value)
+        assert lib.dsqg_linear_wgrad(ctypes.byref(b), None) == _lib.DSQG_EINVAL, field
+
+
+def _pair(dev, I, O, bias, dtype):
+    torch.manual_seed(1)
+    a, b = nn.Linear(I, O, bias=bias), Linear(I, O, bias=bias)
+    b.load_state_dict(a.state_dict(), strict=True)
+    return a.to(dev, dtype), b.to(dev, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["bf16", "f16", "autocast", "autocast_bf16", "f32"])
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("layout", ["plain", "permuted"])
+def test_layer_equals_nn_linear(gpu_device, mode, bias, layout):
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16}.get(mode, torch.float32)
+    low = {"autocast": torch.float16, "autocast_bf16": torch.bfloat16}.get(mode, dtype)
+    ref, lin = _pair(gpu_device, 48, 72, bias, dtype)
+    x = torch.randn(3, 100, 48, device=gpu_device).to(dtype)
+    if layout == "permuted":
+        x = x.permute(1, 0, 2)
+    res = []
+    for m in (ref, lin):
+        xi = x.detach().requires_grad_(True)
+        with torch.amp.autocast("cuda", dtype=low, enabled=mode.startswith("autocast")):
+            y = m(xi)
+        dy = torch.linspace(-1, 1, y.numel(), device=gpu_device).view(y.shape).to(y.dtype)
+        res.append([y.detach(), *torch.autograd.grad(y, [xi, *m.parameters()], dy)])
+    for i, (u, v) in enumerate(zip(*res)):
+        assert u.dtype == v.dtype and u.shape == v.shape
+        if i < 2 or mode == "f32":
+            assert torch.equal(u, v)
+    if mode != "f32":
+        dy2, x2 = dy.reshape(-1, 72), x.to(low).reshape(-1, 48)
+        _close(res[1][2].to(low), dy2, x2, "weight")
+        if bias:
+            _close(res[1][3].to(low), dy2, x2[:, :0], "bias")
+
+
+@pytest.mark.gpu
+def test_layer_keeps_nn_linears_contract(gpu_device):
+    ref, lin = _pair(gpu_device, 48, 72, True, torch.bfloat16)
+    x = torch.randn(64, 48, device=gpu_device).bfloat16().requires_grad_(True)
+    seen = []
+    h = lin.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    # Second derivatives: the gradients are themselves differentiable.
+    (gw,) = torch.autograd.grad(lin(x).float().square().sum(), lin.weight, create_graph=True)
+    (gx,) = torch.autograd.grad(gw.float().sum(), x)
+    w = lin.weight.detach().float()
+    xr = x.detach().float().requires_grad_(True)
+    wr = w.clone().requires_grad_(True)
+    (gwr,) = torch.autograd.grad(F.linear(xr, wr, lin.bias.detach().float()).square().sum(), wr, create_graph=True)
+    (gxr,) = torch.autograd.grad(gwr.sum(), xr)
+    assert (gx.float() - gxr).norm() <= 2e-2 * gxr.norm()
+    h.remove()
+    assert seen == [(64, 72)]
+    lin.bias.requires_grad_(False)
+    (g1,) = torch.autograd.grad(lin(x).float().sum(), lin.weight)
+    lin.weight.requires_grad_(False)
+    assert torch.autograd.grad(lin(x).float().sum(), x)[0].shape == x.shape and g1.shape == (72, 48)
+    with torch.no_grad():
+        assert not lin(x).requires_grad
+    xb = x.detach().view(4, 16, 48)
+    assert torch.equal(torch.vmap(lin)(xb), torch.vmap(ref)(xb))
+    with torch.autograd.forward_ad.dual_level():
+        d = torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x))
+        assert torch.autograd.forward_ad.unpack_dual(lin(d)).tangent is not None
