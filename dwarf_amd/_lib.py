@@ -93,6 +93,14 @@ class PoolBwdArgs(ctypes.Structure):
                 ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t)]
 
 
+class RingLoadArgs(ctypes.Structure):
+    _fields_ = [("dtype", ctypes.c_int32), ("B", ctypes.c_int32), ("H", ctypes.c_int32),
+                ("N", ctypes.c_int32), ("S", ctypes.c_int32), ("D", ctypes.c_int32),
+                ("k", _vp), ("k_stride", ctypes.c_int64 * 3),
+                ("v", _vp), ("v_stride", ctypes.c_int64 * 3),
+                ("k_ring", _vp), ("v_ring", _vp), ("pos", _vp)]
+
+
 class LinearWgradArgs(ctypes.Structure):
     _fields_ = [("T", ctypes.c_int32), ("O", ctypes.c_int32), ("I", ctypes.c_int32),
                 ("dtype", ctypes.c_int32), ("dy", _vp), ("dy_stride", ctypes.c_int64),
@@ -121,6 +129,7 @@ SIGNATURES = {
                                                      ctypes.POINTER(ctypes.c_size_t)]),
     "dsqg_pool_gate_fwd": (ctypes.c_int, [ctypes.POINTER(PoolFwdArgs), _vp]),
     "dsqg_pool_gate_bwd": (ctypes.c_int, [ctypes.POINTER(PoolBwdArgs), _vp]),
+    "dsqg_ring_load": (ctypes.c_int, [ctypes.POINTER(RingLoadArgs), _vp]),
     "dsqg_linear_wgrad_workspace_size": (ctypes.c_int, [ctypes.POINTER(LinearWgradArgs),
                                                         ctypes.POINTER(ctypes.c_size_t)]),
     "dsqg_linear_wgrad": (ctypes.c_int, [ctypes.POINTER(LinearWgradArgs), _vp]),

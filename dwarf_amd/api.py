@@ -213,6 +213,11 @@ class DSQGRingCache:
     def prefill(self, k: Tensor, v: Tensor) -> None:
         """Write prompt rows m = N-S..N-1 (those that exist) to slots m mod S; pos becomes N."""
         B, H, N, D = k.shape
+        state = (self.k_ring, self.v_ring, self.pos)
+        if self.k_ring.is_cuda and not ops.traced(k, v, *state) \
+                and not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)) \
+                and self.S == self.k_ring.shape[2] and _lib.host().ring_load(k, v, *state):
+            return
         lo = max(0, N - self.S)
         idx = torch.arange(lo, N, device=k.device)
         self.k_ring[:, :, idx % self.S] = k[:, :, lo:N].to(self.k_ring.dtype)

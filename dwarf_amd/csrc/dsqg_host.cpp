@@ -33,6 +33,7 @@ struct Api {
   decltype(&dsqg_bwd_workspace_size) bwd_workspace_size = nullptr;
   decltype(&dsqg_bwd) bwd = nullptr;
   decltype(&dsqg_decode_step) decode_step = nullptr;
+  decltype(&dsqg_ring_load) ring_load = nullptr;
   decltype(&dsqg_pool_gate_workspace_size) pool_workspace_size = nullptr;
   decltype(&dsqg_pool_gate_fwd) pool_fwd = nullptr;
   decltype(&dsqg_pool_gate_bwd) pool_bwd = nullptr;
@@ -463,6 +464,44 @@ Tensor decode(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor
   return out;
 }
 
+// Loads k, v [B,H,N,D] into the rings; false (nothing done) where the kernel does not take these
+// tensors as they are: other shapes, types, layouts or devices.
+bool ring_load(const Tensor& k, const Tensor& v, const Tensor& k_ring, const Tensor& v_ring, const Tensor& pos) {
+  py::gil_scoped_release nogil;
+  const auto dt = k_ring.scalar_type();
+  if (!k_ring.is_cuda() || k.dim() != 4 || k_ring.dim() != 4 || v.sizes() != k.sizes() || v_ring.sizes() != k_ring.sizes() ||
+      k.size(0) != k_ring.size(0) || k.size(1) != k_ring.size(1) || k.size(3) != k_ring.size(3) ||
+      (dt != at::kFloat && dt != at::kBFloat16 && dt != at::kHalf) || pos.scalar_type() != at::kLong || pos.dim() != 1 ||
+      pos.size(0) != k.size(0) || !pos.is_contiguous() || !k_ring.is_contiguous() || !v_ring.is_contiguous() || k.numel() == 0)
+    return false;
+  const int64_t es = k.element_size();
+  for (const Tensor* t : {&k, &v}) {
+    if (t->scalar_type() != dt || t->stride(3) != 1) return false;
+    for (int i = 0; i < 3; ++i)
+      if (t->stride(i) < 0 || t->stride(i) * es % 16 != 0) return false;
+  }
+  for (const Tensor* t : {&k, &v, &k_ring, &v_ring, &pos})
+    if (t->device() != k_ring.device() || t->key_set().has(c10::DispatchKey::Python)) return false;
+  for (const Tensor* t : {&k, &v, &k_ring, &v_ring})
+    if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
+  if (k.size(3) * es % 16 != 0 || k.size(0) * k.size(1) > 65535) return false;
+  const c10::OptionalDeviceGuard guard(k_ring.device());
+  dsqg_ring_load_args a = {};
+  a.dtype = dt == at::kFloat ? DSQG_F32 : dt == at::kBFloat16 ? DSQG_BF16 : DSQG_F16;
+  a.B = (int32_t)k.size(0); a.H = (int32_t)k.size(1); a.N = (int32_t)k.size(2); a.D = (int32_t)k.size(3);
+  a.S = (int32_t)k_ring.size(2);
+  a.k = k.data_ptr(); a.v = v.data_ptr();
+  for (int i = 0; i < 3; ++i) { a.k_stride[i] = k.stride(i); a.v_stride[i] = v.stride(i); }
+  a.k_ring = k_ring.data_ptr(); a.v_ring = v_ring.data_ptr();
+  a.pos = static_cast<int64_t*>(pos.data_ptr());
+  const int status = api.ring_load(&a, stream_of(k_ring.device()));
+  if (status == DSQG_EUNSUPPORTED) return false;
+  check(status, "dsqg_ring_load");
+  for (const Tensor* r : {&k_ring, &v_ring, &pos})
+    if (!r->is_inference()) r->unsafeGetTensorImpl()->bump_version();
+  return true;
+}
+
 // ---- Causal-mean pool with a sigmoid gate. ---------------------------------------------------------------------
 
 int pool_code(at::ScalarType dt) { return dt == at::kFloat ? DSQG_F32 : dt == at::kBFloat16 ? DSQG_BF16 : DSQG_F16; }
@@ -640,6 +679,7 @@ void init(const py::dict& addresses, const py::object& library_error) {
   get(api.bwd_workspace_size, "dsqg_bwd_workspace_size");
   get(api.bwd, "dsqg_bwd");
   get(api.decode_step, "dsqg_decode_step");
+  get(api.ring_load, "dsqg_ring_load");
   get(api.pool_workspace_size, "dsqg_pool_gate_workspace_size");
   get(api.pool_fwd, "dsqg_pool_gate_fwd");
   get(api.pool_bwd, "dsqg_pool_gate_bwd");
@@ -656,6 +696,7 @@ PYBIND11_MODULE(_dsqg_host, m) {
   m.def("attention", &attention);
   m.def("attention_qkv", &attention_qkv);
   m.def("decode", &decode);
+  m.def("ring_load", &ring_load);
   m.def("pool_gate", &pool_gate);
   m.def("linear", &linear);
 }

@@ -213,6 +213,24 @@ int dsqg_bwd_noalloc(const dsqg_bwd_args* args, dsqg_stream_t stream);
 
 int dsqg_decode_step(const dsqg_decode_args* args, dsqg_stream_t stream);
 
+/* Loads a prompt into a layer's rings: row m of k and v [B,H,N,D], for m = max(0, N - S) .. N - 1,
+ * goes to slot m mod S of k_ring and v_ring [B,H,S,D] (contiguous; other slots are untouched), and
+ * pos [B] becomes N.  dtype F32, BF16 or F16, of all four; k and v have unit inner stride and the
+ * other strides {b, h, n} and bases keep every row 16-byte aligned; D * sizeof(dtype) is a multiple
+ * of 16 and B * H <= 65535 (EUNSUPPORTED otherwise).  No counterpart in the reference (README.md:
+ * 175-179 describes the ring). */
+typedef struct {
+    int32_t dtype;
+    int32_t B, H, N, S, D;
+    const void* k;  int64_t k_stride[3];
+    const void* v;  int64_t v_stride[3];
+    void* k_ring;
+    void* v_ring;
+    int64_t* pos;
+} dsqg_ring_load_args;
+
+int dsqg_ring_load(const dsqg_ring_load_args* args, dsqg_stream_t stream);
+
 /* Causal-mean pool with a sigmoid gate (the interference branch of a DWARF block):
  *
  *     pool[b,n,c] = (sum_{m<=n} x[b,m,c]) / (n + 1)
