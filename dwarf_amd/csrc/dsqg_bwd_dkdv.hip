@@ -167,11 +167,13 @@ hipError_t launch_bwd_dkdv(const BwdParams& p, int dtype, int D, unsigned nblock
 
 hipError_t launch_bwd_dkdv_params(const BwdParams& p, const ReduceParams& r, int dtype, int D,
                                   unsigned nblocks, hipStream_t st) {
-  if (bwd_mfma_supported(p, D, dtype)) {
+  const bool mfma = bwd_mfma_supported(p, D, dtype);
+  if (mfma || bwd_f32_supported(p, D, dtype)) {
     BwdParams pr = p;
     pr.red = r;
     pr.red_blocks = (int)((reduce_params_waves(r) + kBlock / 64 - 1) / (kBlock / 64));
-    return launch_bwd_dkdv_mfma(pr, D, nblocks + (unsigned)pr.red_blocks, st);
+    nblocks += (unsigned)pr.red_blocks;
+    return mfma ? launch_bwd_dkdv_mfma(pr, D, nblocks, st) : launch_bwd_dkdv_f32(pr, D, nblocks, st);
   }
   const hipError_t e = launch_bwd_dkdv(p, dtype, D, nblocks, st);
   return e != hipSuccess ? e : launch_bwd_reduce_final(r, st);

@@ -12,10 +12,12 @@
 //    wave's key and value rows in the same layout: two row dots, the weights, two row updates.
 // An infinity or NaN among the window's rows would reach other keys through their zero weights:
 // a workgroup that stages one runs every tap as a long-range one (see dsqg_fwd_f32.hip).
-// 33 us at B2 H8 N2047 D64 with scale_embed (the VALU kernel: 52).
+// 34 us at B2 H8 N2047 D64 with scale_embed, the parameter reduction included, which rides in the
+// launch as extra workgroups (apart: 33 + 6.5; the VALU kernel: 52 + 6.5).
 // Follows _bwd_dkdv_v3 (kernels/dsqg_attention_v3.py:282-352), which also needs no atomics.
 #include "dsqg_f32.hpp"
 #include "dsqg_launch.hpp"
+#include "dsqg_reduce.hpp"
 
 namespace dsqg {
 
@@ -36,7 +38,13 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
   __shared__ float sMark[4];
 
   const int tid = threadIdx.x;
-  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  // Workgroups past the dk/dv tiles run the parameter reduction (partials from launch 1).
+  const int kv_blocks = (int)gridDim.x - p.red_blocks;
+  if ((int)blockIdx.x >= kv_blocks) {
+    reduce_params_wave(p.red, ((int)blockIdx.x - kv_blocks) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+    return;
+  }
+  const int lb = xcd_logical_block(blockIdx.x, kv_blocks);
   const int bh = lb / p.n_tiles_kv, tile = lb - bh * p.n_tiles_kv;
   const int b = bh / p.H, h = bh - b * p.H;
   const int N = p.N, J = p.taps.J, W = p.taps.W;
@@ -56,6 +64,11 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
   const bool key_ok = m < N;
 
   // ---- Loads. ----
+  TapParams<D, HAS_SE> tp;
+  tp.load(p.pos_bias, p.score_gain, p.scale_embed, J, p.H, h, tid);
+  const int wrow = tid < WIN ? m0 + tid : N;
+  const float lse_ld = bload1f(rL, wrow), dp_ld = bload1f(rP, wrow);
+  const int dl_lane = p.taps.delta[l < J ? l : 0];
   float4 wq[CWIN], wo[CWIN];
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
@@ -76,7 +89,6 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
     qlane[u] = opaque(rr * qsn + cc);
     olane[u] = opaque(rr * dosn + cc);
   }
-  const int dl_lane = p.taps.delta[l < J ? l : 0];
   int j0 = W + 1;  // first tap taken as a long-range one
   float4 qr[PF][CHW], orr[PF][CHW];
   float lr[PF][RG], pr[PF][RG];
@@ -97,16 +109,9 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
   for (int t = 0; t < PF; ++t)
     if (j0 + t < J) load_tap(j0 + t, t);
 
-  if (tid < kMaxTaps) {
-    const bool in = tid < J;
-    sBias[tid] = in ? p.pos_bias[tid * p.H + h] : 0.f;
-    sGain[tid] = in && p.score_gain ? p.score_gain[h * J + tid] : 1.0f;
-  }
-  if (tid < WIN) {
-    sLse[tid] = bload1f(rL, m0 + tid);
-    sDp[tid] = bload1f(rP, m0 + tid);
-  }
-  if constexpr (HAS_SE) stage_se_f32<D>(sSE, p.scale_embed, J, tid);
+  __builtin_amdgcn_sched_barrier(0);  // (every load above is issued before the first wait)
+  if (tid < WIN) { sLse[tid] = lse_ld; sDp[tid] = dp_ld; }
+  tp.store(sBias, sGain, sSE, J, tid, 0.f);
   float mark = 0.f;
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {

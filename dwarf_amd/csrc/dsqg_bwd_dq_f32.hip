@@ -17,7 +17,7 @@
 // infinity or NaN of a staged K or scale_embed row by other queries' zero weights, so a workgroup
 // that meets one runs every tap as a long-range one (see dsqg_fwd_f32.hip).
 //
-// Bound by latency like the forward: 40 us at B2 H8 N2047 D64 with scale_embed (the VALU kernel:
+// Bound by latency like the forward: 37 us at B2 H8 N2047 D64 with scale_embed (the VALU kernel:
 // 162, with per-tap register arrays it spills, a branch around each long-range load and dse summed
 // one element per thread).
 //
@@ -71,6 +71,10 @@ __global__ __launch_bounds__(kBlock, D <= 64 && !(HAS_SE && DG) ? 2 : 1) void bw
   float* const sR = sRaw + (DG ? w * 16 * TS : 0);
 
   // ---- Loads. ----
+  TapParams<D, HAS_SE> tp;
+  tp.load(p.pos_bias, p.score_gain, p.scale_embed, J, p.H, h, tid);
+  const float lse = p.lse[rowbase + (row_ok ? n : N - 1)];
+  const int dl_lane = p.taps.delta[l < J ? l : 0];
   float4 wk[CWIN], wv[CWIN];
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
@@ -93,8 +97,6 @@ __global__ __launch_bounds__(kBlock, D <= 64 && !(HAS_SE && DG) ? 2 : 1) void bw
     klane[u] = opaque(rr * ksn + cc);
     vlane[u] = opaque(rr * vsn + cc);
   }
-  const float lse = p.lse[rowbase + (row_ok ? n : N - 1)];
-  const int dl_lane = p.taps.delta[l < J ? l : 0];
   int j0 = W + 1;  // first tap taken as a long-range one
   float4 kr[PF][CHW], vr[PF][CHW];
   auto load_k = [&](int j, int slot) {
@@ -111,14 +113,9 @@ __global__ __launch_bounds__(kBlock, D <= 64 && !(HAS_SE && DG) ? 2 : 1) void bw
   for (int t = 0; t < PF; ++t)
     if (j0 + t < J) { load_k(j0 + t, t); load_v(j0 + t, t); }
 
-  if (tid < kMaxTaps) {
-    const bool in = tid < J;
-    sBias[tid] = in ? p.pos_bias[tid * p.H + h] : 0.f;
-    sGain[tid] = in && p.score_gain ? p.score_gain[h * J + tid] : 1.0f;
-    sDelta[tid] = in ? p.taps.delta[tid] : 0;
-  }
-  float mark = 0.f;
-  if constexpr (HAS_SE) mark = stage_se_f32<D>(sSE, p.scale_embed, J, tid);
+  __builtin_amdgcn_sched_barrier(0);  // (every load above is issued before the first wait)
+  if (tid < kMaxTaps) sDelta[tid] = dl_lane;  // (wave 0)
+  float mark = tp.store(sBias, sGain, sSE, J, tid, 0.f);
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
     const int ci = tid + u * kBlock, r = ci / CPR, cc = 4 * (ci - r * CPR);

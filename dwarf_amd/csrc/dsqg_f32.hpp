@@ -128,18 +128,47 @@ __device__ __forceinline__ void lds_wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// scale_embed [J, D] into LDS as 48 rows of stride RV (rows past J zero).
-template <int D>
-__device__ __forceinline__ float stage_se_f32(float* dst, const float* se, int J, int tid) {
-  float mark = 0.f;
-  for (int e = tid; e < kMaxTaps * GeoF<D>::CPR; e += kBlock) {
-    const int j = e / GeoF<D>::CPR, d = 4 * (e - j * GeoF<D>::CPR);
-    const float4 x = se && j < J ? *reinterpret_cast<const float4*>(se + j * D + d) : make_float4(0.f, 0.f, 0.f, 0.f);
-    mark = nonfinite_mark(x, mark);
-    *reinterpret_cast<float4*>(dst + j * GeoF<D>::RV + d) = x;
+// scale_embed [J, D] as 48 rows of stride RV in LDS (rows past J zero), and the per-tap bias and
+// gain: requested ahead of a kernel's bulk loads (load) and stored once the window rows are
+// (store).  Loads return in order, so requested last they would make the first barrier wait for the
+// long-range blocks in flight.
+template <int D, bool HAS_SE>
+struct TapParams {
+  static constexpr int U = HAS_SE ? (kMaxTaps * GeoF<D>::CPR + kBlock - 1) / kBlock : 1;
+  float4 x[U];
+  float bias, gain;
+  __device__ __forceinline__ void load(const float* pos_bias, const float* score_gain, const float* se, int J, int H,
+                                       int h, int tid) {
+    const int jc = tid < J ? tid : J - 1;
+    bias = pos_bias[jc * H + h];
+    gain = score_gain ? score_gain[h * J + jc] : 1.0f;
+    if constexpr (HAS_SE) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = tid + u * kBlock, j = e / GeoF<D>::CPR, d = 4 * (e - j * GeoF<D>::CPR);
+        x[u] = se && j < J ? *reinterpret_cast<const float4*>(se + j * D + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
   }
-  return mark;
-}
+  // Returns mark, made NaN by an infinity or NaN of scale_embed.
+  __device__ __forceinline__ float store(float* sBias, float* sGain, float* sSE, int J, int tid, float mark) const {
+    if (tid < kMaxTaps) {
+      sBias[tid] = tid < J ? bias : 0.f;
+      sGain[tid] = tid < J ? gain : 1.0f;
+    }
+    if constexpr (HAS_SE) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = tid + u * kBlock, j = e / GeoF<D>::CPR, d = 4 * (e - j * GeoF<D>::CPR);
+        if (e < kMaxTaps * GeoF<D>::CPR) {
+          mark = nonfinite_mark(x[u], mark);
+          *reinterpret_cast<float4*>(sSE + j * GeoF<D>::RV + d) = x[u];
+        }
+      }
+    }
+    return mark;
+  }
+};
 
 // Whether every row a kernel touches stays within 32-bit buffer offsets, and rows do not overlap.
 inline bool f32_mfma_strides_ok(int N, int maxd, int D, const long long* rs, int n) {

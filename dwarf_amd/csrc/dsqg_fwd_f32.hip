@@ -20,8 +20,8 @@
 //
 // Bound by latency at the sizes float32 runs at (a 64-row tile is one of two on a CU at B2 H8
 // N2047 D64): what counts is that a tile's loads are all in flight at once and nothing waits per
-// tap.  At that size with scale_embed 27 us for 34 MB read and written
-// (1.2 TB/s); the VALU kernel, whose every tap re-reads its key row from LDS and whose long-range
+// tap.  At that size with scale_embed 25 us for 34 MB read and written
+// (1.3 TB/s); the VALU kernel, whose every tap re-reads its key row from LDS and whose long-range
 // loads sit in a branch each, takes 49.
 //
 // Semantics: _fwd_v3, kernels/dsqg_attention_v3.py:60-163 (plus score gain and IF gain).
@@ -62,7 +62,12 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void fwd_f32_kernel(FwdPar
   const bool row_ok = n < N;
   float* const sT = sTab[w];
 
-  // ---- Loads: window, query rows in both layouts, the first long-range key rows. ----
+  // ---- Loads: per-tap parameters, window, query rows in both layouts, the first long-range key
+  // rows. ----
+  TapParams<D, HAS_SE> tp;
+  tp.load(p.pos_bias, p.score_gain, p.scale_embed, J, p.H, h, tid);
+  const float if_a = p.if_gain ? p.if_gain[h] : 1.0f;
+  const int dl_lane = p.taps.delta[l < J ? l : 0];  // lane j holds tap j's offset
   float4 wk[CWIN], wv[CWIN];
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
@@ -81,7 +86,6 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void fwd_f32_kernel(FwdPar
     klane[u] = opaque(rf_row<D>(l, u) * ksn + rf_col<D>(l, u));
     vlane[u] = opaque(rf_row<D>(l, u) * vsn + rf_col<D>(l, u));
   }
-  const int dl_lane = p.taps.delta[l < J ? l : 0];  // lane j holds tap j's offset
   int j0 = W + 1;                                   // first tap taken as a long-range one
   float4 ring[PF][CHW];
   auto load_k = [&](int j, int slot) {
@@ -98,13 +102,9 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void fwd_f32_kernel(FwdPar
   for (int t = 0; t < PF; ++t)
     if (j0 + t < J) load_k(j0 + t, t);
 
-  if (tid < kMaxTaps) {
-    const bool in = tid < J;
-    sBias[tid] = in ? p.pos_bias[tid * p.H + h] : 0.f;
-    sGain[tid] = in && p.score_gain ? p.score_gain[h * J + tid] : 1.0f;
-    sDelta[tid] = in ? p.taps.delta[tid] : 0;
-  }
-  if constexpr (HAS_SE) stage_se_f32<D>(sSE, p.scale_embed, J, tid);
+  __builtin_amdgcn_sched_barrier(0);  // (every load above is issued before the first wait)
+  if (tid < kMaxTaps) sDelta[tid] = dl_lane;  // (wave 0)
+  tp.store(sBias, sGain, sSE, J, tid, 0.f);
   float mark = 0.f;
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void fwd_f32_kernel(FwdPar
   }
   lsum = col_sum(lsum);
   if (row_ok && g == 0 && p.lse) p.lse[(long long)bh * N + n] = mx + __logf(lsum);
-  if (g == 0) sInv[w][i] = (p.if_gain ? p.if_gain[h] : 1.0f) / lsum;
+  if (g == 0) sInv[w][i] = if_a / lsum;
 
   // ---- Band P V, O^T = V^T P^T. ----
   f32x4_t O[DB];
