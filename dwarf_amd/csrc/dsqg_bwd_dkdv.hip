@@ -171,12 +171,13 @@ hipError_t launch_bwd_dkdv_params(const BwdParams& p, const ReduceParams& r, int
   if (mfma || bwd_f32_supported(p, D, dtype)) {
     BwdParams pr = p;
     pr.red = r;
-    pr.red_blocks = (int)((reduce_params_waves(r) + kBlock / 64 - 1) / (kBlock / 64));
-    nblocks += (unsigned)pr.red_blocks;
+    pr.red_se_blocks = reduce_se_blocks(r);
+    pr.red_blocks = reduce_wave_blocks(r);
+    nblocks += (unsigned)(pr.red_se_blocks + pr.red_blocks);
     return mfma ? launch_bwd_dkdv_mfma(pr, D, nblocks, st) : launch_bwd_dkdv_f32(pr, D, nblocks, st);
   }
   const hipError_t e = launch_bwd_dkdv(p, dtype, D, nblocks, st);
-  return e != hipSuccess ? e : launch_bwd_reduce_final(r, st);
+  return e != hipSuccess ? e : launch_bwd_reduce(r, st);
 }
 
 }  // namespace dsqg

@@ -38,13 +38,18 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
   __shared__ float sMark[4];
 
   const int tid = threadIdx.x;
-  // Workgroups past the dk/dv tiles run the parameter reduction (partials from launch 1).
-  const int kv_blocks = (int)gridDim.x - p.red_blocks;
-  if ((int)blockIdx.x >= kv_blocks) {
-    reduce_params_wave(p.red, ((int)blockIdx.x - kv_blocks) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+  // Workgroups before and past the dk/dv tiles run the parameter reduction (partials from launch 1).
+  const int bid = (int)blockIdx.x - p.red_se_blocks;
+  if (bid < 0) {
+    reduce_se_block(p.red, (int)blockIdx.x, tid, sQ);
     return;
   }
-  const int lb = xcd_logical_block(blockIdx.x, kv_blocks);
+  const int kv_blocks = (int)gridDim.x - p.red_se_blocks - p.red_blocks;
+  if (bid >= kv_blocks) {
+    reduce_params_wave(p.red, (bid - kv_blocks) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+    return;
+  }
+  const int lb = xcd_logical_block(bid, kv_blocks);
   const int bh = lb / p.n_tiles_kv, tile = lb - bh * p.n_tiles_kv;
   const int b = bh / p.H, h = bh - b * p.H;
   const int N = p.N, J = p.taps.J, W = p.taps.W;

@@ -28,8 +28,9 @@
 //    on the MFMA (Q SE^T) with se rounded to bf16 (an error of about 2^-9 |c q.se| in the score,
 //    1e-4 at the reference's se ~ 0.05; the parameter gradients come from launch 1, which keeps
 //    se at fp32 precision).
-// With p.red_blocks > 0 the launch carries that many extra workgroups at the end of the grid,
-// which sum the parameter-gradient partials (dsqg_reduce.hpp) while the dk/dv tiles run.
+// In a full backward the launch carries extra workgroups that sum the parameter-gradient partials
+// (dsqg_reduce.hpp) while the dk/dv tiles run: dscale_embed's at the start of the grid, the others
+// at its end.
 // Follows _bwd_dkdv_v3 (kernels/dsqg_attention_v3.py:282-352).
 #include "dsqg_common.hpp"
 #include "dsqg_launch.hpp"
@@ -80,10 +81,15 @@ __global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 && HAS_SE ? 3 : 4)) 
   __shared__ float sGainC[HAS_SE ? 1 : kMaxTaps];    // gain * c (with scale_embed: sGain2 ln 2)
 
   const int tid = threadIdx.x;
-  // Workgroups past the dk/dv tiles run the parameter reduction (partials from launch 1).
-  const int kv_blocks = (int)gridDim.x - p.red_blocks;
-  if ((int)blockIdx.x >= kv_blocks) {
-    reduce_params_wave(p.red, ((int)blockIdx.x - kv_blocks) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+  // Workgroups before and past the dk/dv tiles run the parameter reduction (partials from launch 1).
+  const int bid = (int)blockIdx.x - p.red_se_blocks;
+  if (bid < 0) {
+    reduce_se_block(p.red, (int)blockIdx.x, tid, reinterpret_cast<float*>(sQO));
+    return;
+  }
+  const int kv_blocks = (int)gridDim.x - p.red_se_blocks - p.red_blocks;
+  if (bid >= kv_blocks) {
+    reduce_params_wave(p.red, (bid - kv_blocks) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
     return;
   }
   // The kernel arguments of the prologue in one round trip: sizes and input strides pass through
@@ -96,7 +102,7 @@ __global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 && HAS_SE ? 3 : 4)) 
                "+s"(p.vs.b), "+s"(p.vs.h), "+s"(p.vs.n), "+s"(p.dos.b), "+s"(p.dos.h), "+s"(p.dos.n)
                : "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.dout), "s"(p.lse), "s"(p.dpre), "s"(p.pos_bias),
                  "s"(p.if_gain));
-  const int lb = xcd_logical_block(blockIdx.x, kv_blocks);
+  const int lb = xcd_logical_block(bid, kv_blocks);
   const int bh = lb / p.n_tiles_kv, tile = lb - bh * p.n_tiles_kv;
   const int b = bh / p.H, h = bh - b * p.H;
   const int N = p.N, J = p.taps.J, W = p.taps.W;

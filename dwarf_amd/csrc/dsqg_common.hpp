@@ -145,9 +145,6 @@ struct ReduceParams {
   int B, H, J, D, n_chunks;  // B: batch groups of the partials (BwdParams::n_bgroups)
   const float* part_bias; const float* part_se; const float* part_gain; const float* part_if;
   float* dpos_bias; float* dscale_embed; float* dscore_gain; float* dif_gain;
-  // dscale_embed is summed in two stages: se_slices runs of se_per consecutive workgroup
-  // partials each, summed column-wise into se_stage [se_slices][J*D], then the slices.
-  float* se_stage; int se_slices, se_per;
 };
 
 struct BwdParams {
@@ -185,9 +182,10 @@ struct BwdParams {
   // low half bf16(c g_j dS_j) (the weight of q_n in dk), high half bf16(a alpha_j) (the weight
   // of dOut_n in dv).
   float* lrw;
-  // Parameter reduction run by red_blocks extra workgroups of the bf16 dk/dv launch (0: none).
+  // Parameter reduction run by extra workgroups of the MFMA dk/dv launches: red_se_blocks before
+  // the tiles (dscale_embed) and red_blocks after them (the rest); 0: none.
   ReduceParams red;
-  int red_blocks;
+  int red_se_blocks, red_blocks;
 };
 
 

@@ -1,6 +1,7 @@
-// Parameter-gradient reduction (dbias, dscore_gain, dif_gain, dscale_embed's final stage), one
-// wave per output element: shared by bwd_reduce_kernel (dsqg_bwd.hip) and the extra workgroups
-// of the bf16 dk/dv launch (dsqg_bwd_dkdv_mfma.hip), which run it next to the dk/dv tiles.
+// Parameter-gradient reduction (dbias, dscore_gain and dif_gain one wave per output element,
+// dscale_embed a workgroup per 32 elements): shared by bwd_reduce_kernel (dsqg_bwd.hip) and the extra workgroups
+// of the MFMA dk/dv launches (dsqg_bwd_dkdv_mfma.hip, dsqg_bwd_dkdv_f32.hip), which run it next to
+// the dk/dv tiles.
 #pragma once
 
 #include "dsqg_common.hpp"
@@ -57,18 +58,48 @@ __device__ __forceinline__ void reduce_params_wave(const ReduceParams& r, int t,
     }
     t -= r.H;
   }
-  if (r.dscale_embed && t < r.J * r.D) {
-    const long long stride = (long long)r.J * r.D;
+}
+
+// dscale_embed: workgroup blk sums the partials of 32 consecutive elements of [J*D].  A thread
+// takes four of them (16 bytes; eight lanes read 128 contiguous bytes) of every 32nd partial row,
+// eight rows in flight, and the 32 row sums of an element meet in LDS in order.  lds: 32 x 32
+// floats.  At the start of the dk/dv grid these few workgroups finish long before its tiles do; as
+// a launch of its own between dq and dk/dv (a first stage of 256 slices) the sum cost 5 us.
+constexpr int kSeGroup = 32;
+
+__device__ __forceinline__ void reduce_se_block(const ReduceParams& r, int blk, int tid, float* lds) {
+  const int JD = r.J * r.D;  // a multiple of 16
+  const int c = 4 * (tid & 7), row = tid >> 3;
+  const int e = blk * kSeGroup + c;
+  const int rows = r.B * r.H * r.n_chunks;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (e < JD) {
+    const float* src = r.part_se + e;
+#pragma unroll 8
+    for (int k = row; k < rows; k += kBlock / 8) {
+      const float4 x = *reinterpret_cast<const float4*>(src + (long long)k * JD);
+      acc.x += x.x; acc.y += x.y; acc.z += x.z; acc.w += x.w;
+    }
+  }
+  *reinterpret_cast<float4*>(lds + row * kSeGroup + c) = acc;
+  __syncthreads();
+  if (tid < kSeGroup && blk * kSeGroup + tid < JD) {
     float s = 0.f;
-    for (int k = lane; k < r.se_slices; k += 64) s += r.se_stage[k * stride + t];
-    s = wave_sum_fixed(s);
-    if (lane == 0) r.dscale_embed[t] = s;
+#pragma unroll
+    for (int k = 0; k < kBlock / 8; ++k) s += lds[k * kSeGroup + tid];
+    r.dscale_embed[blk * kSeGroup + tid] = s;
   }
 }
 
-// Waves needed for every output of r (an upper bound; surplus waves return at once).
-inline long long reduce_params_waves(const ReduceParams& r) {
-  return 2LL * r.J * r.H + r.H + (long long)r.J * r.D;
+// Workgroups of the two parts: dscale_embed's (a multiple of the XCD count, so that the workgroups
+// after them keep their XCDs) and the one-wave-per-element rest (an upper bound; surplus waves
+// return at once).
+inline int reduce_se_blocks(const ReduceParams& r) {
+  if (!r.dscale_embed) return 0;
+  return ((r.J * r.D + kSeGroup - 1) / kSeGroup + kNumXcd - 1) / kNumXcd * kNumXcd;
+}
+inline int reduce_wave_blocks(const ReduceParams& r) {
+  return (int)((2LL * r.J * r.H + r.H + kBlock / 64 - 1) / (kBlock / 64));
 }
 
 }  // namespace dsqg
