@@ -93,6 +93,16 @@ class PoolBwdArgs(ctypes.Structure):
                 ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t)]
 
 
+class KvInjectArgs(ctypes.Structure):
+    _fields_ = [("B", ctypes.c_int32), ("H", ctypes.c_int32), ("N", ctypes.c_int32),
+                ("D", ctypes.c_int32), ("qkv_dtype", ctypes.c_int32),
+                ("delta_dtype", ctypes.c_int32), ("out_dtype", ctypes.c_int32),
+                ("qkv", _vp), ("qkv_stride", _i64x2),
+                ("k_delta", _vp), ("k_delta_stride", ctypes.c_int64 * 3),
+                ("v_delta", _vp), ("v_delta_stride", ctypes.c_int64 * 3),
+                ("q_out", _vp), ("k_out", _vp), ("v_out", _vp), ("out_stride", _i64x2)]
+
+
 class RingLoadArgs(ctypes.Structure):
     _fields_ = [("dtype", ctypes.c_int32), ("B", ctypes.c_int32), ("H", ctypes.c_int32),
                 ("N", ctypes.c_int32), ("S", ctypes.c_int32), ("D", ctypes.c_int32),
@@ -129,6 +139,7 @@ SIGNATURES = {
                                                      ctypes.POINTER(ctypes.c_size_t)]),
     "dsqg_pool_gate_fwd": (ctypes.c_int, [ctypes.POINTER(PoolFwdArgs), _vp]),
     "dsqg_pool_gate_bwd": (ctypes.c_int, [ctypes.POINTER(PoolBwdArgs), _vp]),
+    "dsqg_kv_inject": (ctypes.c_int, [ctypes.POINTER(KvInjectArgs), _vp]),
     "dsqg_ring_load": (ctypes.c_int, [ctypes.POINTER(RingLoadArgs), _vp]),
     "dsqg_linear_wgrad_workspace_size": (ctypes.c_int, [ctypes.POINTER(LinearWgradArgs),
                                                         ctypes.POINTER(ctypes.c_size_t)]),

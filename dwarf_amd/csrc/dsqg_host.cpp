@@ -33,6 +33,7 @@ struct Api {
   decltype(&dsqg_bwd_workspace_size) bwd_workspace_size = nullptr;
   decltype(&dsqg_bwd) bwd = nullptr;
   decltype(&dsqg_decode_step) decode_step = nullptr;
+  decltype(&dsqg_kv_inject) kv_inject = nullptr;
   decltype(&dsqg_ring_load) ring_load = nullptr;
   decltype(&dsqg_pool_gate_workspace_size) pool_workspace_size = nullptr;
   decltype(&dsqg_pool_gate_fwd) pool_fwd = nullptr;
@@ -317,35 +318,82 @@ struct AttentionQkvFunction : torch::autograd::Function<AttentionQkvFunction> {
   }
 };
 
+// The attended operands of a K/V injection: q, K + k_delta and V + v_delta as [B,H,N,HD] views, in
+// the compute type dt.
+struct Injected {
+  Tensor q, k, v;
+};
+
+Injected inject(const Tensor& qkv, const Tensor& kd, const Tensor& vd, int64_t H, at::ScalarType dt) {
+  const int64_t B = qkv.size(0), N = qkv.size(1), E = qkv.size(2) / 3, HD = E / H;
+  const bool cast = qkv.scalar_type() != dt;
+  auto aligned = [](const Tensor& t) {
+    bool ok = t.stride(t.dim() - 1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    for (int64_t i = 0; ok && i < t.dim() - 1; ++i) ok = t.stride(i) >= 0 && t.stride(i) * t.element_size() % 16 == 0;
+    return ok;
+  };
+  // What the kernel takes; anything else is the casts and adds one by one.
+  if (qkv.numel() == 0 || HD % 8 != 0 || E * qkv.element_size() % 16 != 0 || kd.scalar_type() != qkv.scalar_type() ||
+      vd.scalar_type() != qkv.scalar_type() || !kd.is_cuda() || !vd.is_cuda() || !qkv.is_cuda() ||
+      kd.device() != qkv.device() || vd.device() != qkv.device() || (cast && qkv.scalar_type() != at::kHalf) ||
+      !aligned(qkv) || !aligned(kd) || !aligned(vd)) {
+    const Tensor x = qkv.to(dt);
+    return {head_view(x, H, 0), head_view(x, H, 1) + kd.to(dt), head_view(x, H, 2) + vd.to(dt)};
+  }
+  const c10::OptionalDeviceGuard guard(qkv.device());
+  const int64_t parts = cast ? 3 : 2;  // q is read from qkv itself where the types agree
+  const Tensor eff = at::empty({B, N, parts * E}, qkv.options().dtype(dt));
+  auto view = [&](int64_t part) {
+    return eff.as_strided({B, H, N, HD}, {N * parts * E, HD, parts * E, 1}, part * E);
+  };
+  Injected r{cast ? view(0) : head_view(qkv, H, 0), view(parts - 2), view(parts - 1)};
+  auto code = [](at::ScalarType t) { return t == at::kFloat ? DSQG_F32 : t == at::kBFloat16 ? DSQG_BF16 : DSQG_F16; };
+  dsqg_kv_inject_args a = {};
+  a.B = (int32_t)B; a.H = (int32_t)H; a.N = (int32_t)N; a.D = (int32_t)HD;
+  a.qkv_dtype = a.delta_dtype = code(qkv.scalar_type());
+  a.out_dtype = code(dt);
+  a.qkv = qkv.data_ptr(); a.qkv_stride[0] = qkv.stride(0); a.qkv_stride[1] = qkv.stride(1);
+  a.k_delta = kd.data_ptr(); a.v_delta = vd.data_ptr();
+  for (int i = 0; i < 3; ++i) { a.k_delta_stride[i] = kd.stride(i); a.v_delta_stride[i] = vd.stride(i); }
+  a.q_out = cast ? r.q.data_ptr() : nullptr;
+  a.k_out = r.k.data_ptr(); a.v_out = r.v.data_ptr();
+  a.out_stride[0] = N * parts * E; a.out_stride[1] = parts * E;
+  check(api.kv_inject(&a, stream_of(qkv.device())), "dsqg_kv_inject");
+  return r;
+}
+
 // The same with a K/V injection: K + k_delta and V + v_delta are attended, and the K and V slices
-// of d(qkv) are also the deltas' gradients.
+// of d(qkv) are also the deltas' gradients.  Takes qkv in its own type (dt: the compute type).
 struct AttentionQkvKvFunction : torch::autograd::Function<AttentionQkvKvFunction> {
   static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& kd, const Tensor& vd,
                                const Tensor& pb, const OptTensor& se, const OptTensor& sg, const OptTensor& ig,
-                               int64_t H, const TablePtr& t) {
-    const auto dt = qkv.scalar_type();
-    const Tensor k = head_view(qkv, H, 1) + kd.to(dt), v = head_view(qkv, H, 2) + vd.to(dt);
-    const FwdOut r = run_fwd(head_view(qkv, H, 0), k, v, {pb, undef(se), undef(sg), undef(ig)}, *t);
-    ctx->save_for_backward({qkv, k, v, r.lse, r.alpha_lr, pb, undef(se), undef(sg), undef(ig)});
+                               int64_t H, at::ScalarType dt, const TablePtr& t) {
+    require_gpu({&qkv, &kd, &vd});
+    const Injected x = inject(qkv, kd, vd, H, dt);
+    const FwdOut r = run_fwd(x.q, x.k, x.v, {pb, undef(se), undef(sg), undef(ig)}, *t);
+    ctx->save_for_backward({x.q, x.k, x.v, r.lse, r.alpha_lr, pb, undef(se), undef(sg), undef(ig)});
     ctx->saved_data["table"] = c10::IValue::make_capsule(t);
-    ctx->saved_data["H"] = H;
-    ctx->saved_data["kd"] = (int64_t)kd.scalar_type();
-    ctx->saved_data["vd"] = (int64_t)vd.scalar_type();
-    ctx->mark_non_differentiable({r.lse, r.alpha_lr, k, v});
-    return {r.out, r.lse, r.alpha_lr, k, v};
+    ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)qkv.scalar_type(), (int64_t)kd.scalar_type(),
+                                                    (int64_t)vd.scalar_type()};
+    ctx->mark_non_differentiable({r.lse, r.alpha_lr});
+    return {r.out, r.lse, r.alpha_lr};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
-    const int64_t H = ctx->saved_data["H"].toInt();
+    const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
     const Params P{s[5], s[6], s[7], s[8]};
     const Needs n(ctx, {true, true, true, true, P.se.defined(), P.sg.defined(), P.ig.defined()});
-    const Tensor dqkv = at::empty_like(s[0], at::MemoryFormat::Contiguous);
+    const int64_t B = s[0].size(0), H = s[0].size(1), N = s[0].size(2), HD = s[0].size(3);
+    const Tensor dqkv = at::empty({B, N, 3 * H * HD}, s[0].options());
     Grads G;
     G.dq = head_view(dqkv, H, 0); G.dk = head_view(dqkv, H, 1); G.dv = head_view(dqkv, H, 2);
-    run_bwd(G, head_view(s[0], H, 0), s[1], s[2], g[0], s[3], s[4], P, table_of(ctx), n.need[4], n.need[5],
-            n.need[6]);
-    return {dqkv, G.dk.to((at::ScalarType)ctx->saved_data["kd"].toInt()),
-            G.dv.to((at::ScalarType)ctx->saved_data["vd"].toInt()), G.dpb, G.dse, G.dsg, G.dig, Tensor(), Tensor()};
+    run_bwd(G, s[0], s[1], s[2], g[0], s[3], s[4], P, table_of(ctx), n.need[4], n.need[5], n.need[6]);
+    // One cast of the whole gradient; a delta of qkv's type takes its slice of the result.
+    const Tensor dx = dqkv.to((at::ScalarType)types[0]);
+    auto delta = [&](int part) {
+      return types[part] == types[0] ? head_view(dx, H, part) : head_view(dqkv, H, part).to((at::ScalarType)types[part]);
+    };
+    return {dx, delta(1), delta(2), G.dpb, G.dse, G.dsg, G.dig, Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -403,15 +451,15 @@ Tensor attention_qkv(const Tensor& qkv0, int64_t H, const Tensor& pb, const OptT
   expect(undef(sg), {H, t->J}, "score_gain");
   expect(undef(ig), {H}, "if_gain");
   const auto orig = qkv0.scalar_type();
-  const Tensor qkv = kernel_dtype(orig) ? qkv0 : qkv0.to(at::kBFloat16);
+  const auto dt = kernel_dtype(orig) ? orig : at::kBFloat16;
   const Params P = float_params(pb, se, sg, ig);
   variable_list r;
   if (!kd.has_value()) {
-    r = AttentionQkvFunction::apply(qkv, P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, t);
+    r = AttentionQkvFunction::apply(qkv0.to(dt), P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, t);
   } else {
     require(kd->sizes() == c10::IntArrayRef(heads) && vd->sizes() == c10::IntArrayRef(heads),
             "kv_inject deltas must be torch.Size([", heads[0], ", ", heads[1], ", ", heads[2], ", ", heads[3], "])");
-    r = AttentionQkvKvFunction::apply(qkv, *kd, *vd, P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, t);
+    r = AttentionQkvKvFunction::apply(qkv0, *kd, *vd, P.pb, opt(P.se), opt(P.sg), opt(P.ig), H, dt, t);
   }
   return r[0].to(orig);
 }
@@ -679,6 +727,7 @@ void init(const py::dict& addresses, const py::object& library_error) {
   get(api.bwd_workspace_size, "dsqg_bwd_workspace_size");
   get(api.bwd, "dsqg_bwd");
   get(api.decode_step, "dsqg_decode_step");
+  get(api.kv_inject, "dsqg_kv_inject");
   get(api.ring_load, "dsqg_ring_load");
   get(api.pool_workspace_size, "dsqg_pool_gate_workspace_size");
   get(api.pool_fwd, "dsqg_pool_gate_fwd");

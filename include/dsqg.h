@@ -213,6 +213,26 @@ int dsqg_bwd_noalloc(const dsqg_bwd_args* args, dsqg_stream_t stream);
 
 int dsqg_decode_step(const dsqg_decode_args* args, dsqg_stream_t stream);
 
+/* K/V injection before the attention (train/train_2048_condU.py:178-181): with qkv [B,N,3*H*D] (unit
+ * inner stride, element strides {b, n}) and deltas [B,H,N,D] (unit inner stride, strides {b, h, n}),
+ * k_out = k + k_delta and v_out = v + v_delta, and q_out = q when given, each [B,N,H*D] with the
+ * strides out_stride {b, n}; operands are rounded to out_dtype before the sum.  Types taken: all
+ * F32, all BF16, or F16 in and BF16 out (EUNSUPPORTED otherwise).  D is a multiple of 8; bases and
+ * strides keep every row 16-byte aligned. */
+typedef struct {
+    int32_t B, H, N, D;
+    int32_t qkv_dtype, delta_dtype, out_dtype;
+    const void* qkv;      int64_t qkv_stride[2];
+    const void* k_delta;  int64_t k_delta_stride[3];
+    const void* v_delta;  int64_t v_delta_stride[3];
+    void* q_out;          /* or NULL */
+    void* k_out;
+    void* v_out;
+    int64_t out_stride[2];
+} dsqg_kv_inject_args;
+
+int dsqg_kv_inject(const dsqg_kv_inject_args* args, dsqg_stream_t stream);
+
 /* Loads a prompt into a layer's rings: row m of k and v [B,H,N,D], for m = max(0, N - S) .. N - 1,
  * goes to slot m mod S of k_ring and v_ring [B,H,S,D] (contiguous; other slots are untouched), and
  * pos [B] becomes N.  dtype F32, BF16 or F16, of all four; k and v have unit inner stride and the
