@@ -47,7 +47,7 @@ constexpr int kDqTableStride = 52;
 // DG: the score gain's gradient is requested (its c q.k table in dynamic LDS and the extra row
 // sums are compiled in only then).
 template <int D, bool HAS_SE, int NSC, bool DG>
-__global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 || (HAS_SE && NSC != 11) ? 2 : (HAS_SE || DG ? 3 : 4)))
+__global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 || (HAS_SE && NSC != 11 && D > 32) ? 2 : ((HAS_SE && D > 32) || DG ? 3 : 4)))
 void bwd_dq_mfma_kernel(BwdParams p) {
   using G_ = Geo<D>;
   constexpr int QT = 64;
@@ -65,8 +65,8 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   // Long-range row blocks loaded ahead of use: as many as the register budget of the occupancy
   // target holds without spills (a tap is a few dozen VALU instructions per wave).  Four in the
   // plain 11-tap form; two above D = 64, in the scale_embed forms other than the 11-tap one
-  // without the gain's gradient, and in the plain generic-table form; three otherwise.
-  constexpr int PF = (D > 64 || (HAS_SE && (NSC != 11 || DG)) || (NSC == 0 && !DG))
+  // without the gain's gradient at D = 64, and in the plain generic-table form; three otherwise.
+  constexpr int PF = (D > 64 || (HAS_SE && (D == 32 || NSC != 11 || DG)) || (NSC == 0 && !DG))
                          ? 2
                          : (HAS_SE || DG || NSC != 11 ? 3 : 4);
   constexpr int TS = kDqTableStride;
@@ -79,11 +79,21 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   constexpr float kLog2e = 1.4426950408889634f;
 
   __shared__ __align__(16) bf16_t sK[WIN * RV];        // dense-window K rows
-  __shared__ __align__(16) bf16_t sV[WIN * RV];        // dense-window V rows
+  // At D = 32 with scale_embed the per-wave tables do not fit the V window alone, and with tables
+  // of their own (46.7 KB) three workgroups fit a CU: one region holds the V window and the T
+  // tables during the band, then the [query][tap] tables and the staging blocks (34.4 KB), and
+  // four fit.  B8 H8 N2048 with 11 long-range taps: 42.1 -> 35.6 us (two batches each; B16 76 ->
+  // 62 with four).
+  constexpr bool PACKED = HAS_SE && D == 32;
+  constexpr int TBL_B = 4 * 16 * TS * 2;               // bf16 elements of the tables
+  static_assert(!PACKED || (WIN * RV <= TBL_B && 4 * 32 * TST <= TBL_B + 4 * 16 * RV - WIN * RV), "phases fit");
+  __shared__ __align__(16) bf16_t sV[PACKED ? TBL_B + 4 * 16 * RV : WIN * RV];  // dense-window V rows
   // Wave-private staging block: with scale_embed first the dense-tap table
   // T[i][j] = log2e (bias_j + c q_i.se_j); then the two rounds that turn dq into row layout;
   // then, with scale_embed, the wave's Q rows (read by every wave for dse).
-  __shared__ __align__(16) bf16_t sKs[4][HAS_SE ? KSB : 16 * RV];
+  __shared__ __align__(16) bf16_t sKsst[PACKED ? 8 : 4 * (HAS_SE ? KSB : 16 * RV)];
+  constexpr int KST = PACKED || !HAS_SE ? 16 * RV : KSB;  // elements of a wave's block
+  bf16_t* const sKs = PACKED ? sV + TBL_B : sKsst;
   // scale_embed rows as two bf16 planes, hi = bf16(se) and lo = bf16(se - hi): q.se and
   // SE^T dS then carry se to about 2^-17 relative, as the fp32 se of the reference.
   __shared__ __align__(16) bf16_t sSE[HAS_SE ? SEJ * RV : 8];
@@ -91,7 +101,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   // [query][tap] per wave: u of the long-range taps (pass 1), then dS.  It lives in the V window
   // once the band is done (D >= 64), which keeps the workgroup's LDS small enough for four
   // workgroups per CU (three with scale_embed).
-  constexpr bool TBL_IN_V = WIN * RV * 2 >= 4 * 16 * TS * 4;
+  constexpr bool TBL_IN_V = PACKED || WIN * RV * 2 >= 4 * 16 * TS * 4;
   __shared__ __align__(16) float sDSst[TBL_IN_V ? 4 : 4 * 16 * TS];
   // c q.k per (query, tap), for dg only: dynamic LDS, present when score_gain's gradient is
   // requested.
@@ -161,8 +171,8 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   }
   float* sDSw = sDS + w * 16 * TS;
   float* sRAWw = sRAW + w * 16 * TS;  // dereferenced only when g_grad
-  bf16_t* sKsw = sKs[w];
-  float* sTw = reinterpret_cast<float*>(sKsw);
+  bf16_t* sKsw = sKs + w * KST;
+  float* sTw = reinterpret_cast<float*>(PACKED ? sV + WIN * RV + w * 32 * TST : sKsw);
 
   // The parameter-gradient partials of the workgroup's (b,h) slices, summed in batch order.  With
   // scale_embed a workgroup takes its head and tile in p.batches_per_block batches, so that its
@@ -459,7 +469,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
     constexpr int HC = G_::DP / 2;  // columns per round
     constexpr int CS = HC + 4;
     constexpr int CPH = HC / 8;     // row chunks per round
-    static_assert(16 * CS * 4 <= (HAS_SE ? KSB : 16 * RV) * 2, "a round fits the staging block");
+    static_assert(16 * CS * 4 <= KST * 2, "a round fits the staging block");
     float* const cvt = reinterpret_cast<float*>(sKsw);
 #pragma unroll
     for (int u = 0; u < CHW; ++u)
@@ -584,7 +594,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
             const float* col = sDS + (ww * 16 + 4 * g) * TS + 16 * jb + i;
             s16x4_t bs, bsl;
             split_bf16x4(col[0], col[TS], col[2 * TS], col[3 * TS], bs, bsl);
-            const bf16_t* qr = sKs[ww] + (4 * g + (i >> 2)) * RV + 4 * (i & 3) + 16 * db;
+            const bf16_t* qr = sKs + ww * KST + (4 * g + (i >> 2)) * RV + 4 * (i & 3) + 16 * db;
             const s16x4_t qt = lds_read_tr16(qr);
             accSE[k] = mfma_16x16x16(qt, bs, accSE[k]);
             accSE[k] = mfma_16x16x16(qt, bsl, accSE[k]);
