@@ -113,7 +113,7 @@ class RingLoadArgs(ctypes.Structure):
 
 class LinearWgradArgs(ctypes.Structure):
     _fields_ = [("T", ctypes.c_int32), ("O", ctypes.c_int32), ("I", ctypes.c_int32),
-                ("dtype", ctypes.c_int32), ("dy", _vp), ("dy_stride", ctypes.c_int64),
+                ("dtype", ctypes.c_int32), ("out_dtype", ctypes.c_int32), ("dy", _vp), ("dy_stride", ctypes.c_int64),
                 ("x", _vp), ("x_stride", ctypes.c_int64), ("dw", _vp), ("db", _vp),
                 ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t)]
 

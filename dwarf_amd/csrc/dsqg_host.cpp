@@ -647,15 +647,16 @@ Tensor wgrad_rows(const Tensor& t) {
   return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
-void linear_wgrad(const Tensor& dy0, const Tensor& x0, bool need_db, Tensor& dw, Tensor& db) {
+void linear_wgrad(const Tensor& dy0, const Tensor& x0, at::ScalarType out, bool need_db, Tensor& dw, Tensor& db) {
   const c10::Device dev = require_gpu({&dy0, &x0});
   const c10::OptionalDeviceGuard guard(dev);
   const Tensor dy = wgrad_rows(dy0), x = wgrad_rows(x0);
-  dw = at::empty({dy.size(1), x.size(1)}, x.options());
-  if (need_db) db = at::empty({dy.size(1)}, x.options());
+  dw = at::empty({dy.size(1), x.size(1)}, x.options().dtype(out));
+  if (need_db) db = at::empty({dy.size(1)}, x.options().dtype(out));
   dsqg_linear_wgrad_args a = {};
   a.T = (int32_t)dy.size(0); a.O = (int32_t)dy.size(1); a.I = (int32_t)x.size(1);
   a.dtype = pool_code(x.scalar_type());
+  a.out_dtype = pool_code(out);
   a.dy = dy.data_ptr(); a.dy_stride = dy.stride(0);
   a.x = x.data_ptr(); a.x_stride = x.stride(0);
   a.dw = dw.data_ptr();
@@ -667,55 +668,57 @@ void linear_wgrad(const Tensor& dy0, const Tensor& x0, bool need_db, Tensor& dw,
   check(api.linear_wgrad(&a, stream_of(dev)), "dsqg_linear_wgrad");
 }
 
+// x in the compute type; w and b in it too, or the float32 parameters autocast would cast: then the
+// casts happen here and their gradients come out of the kernel in float32.
 struct LinearFunction : torch::autograd::Function<LinearFunction> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& b) {
-    ctx->save_for_backward({x, w});
-    ctx->saved_data["bias"] = b.has_value();
-    return at::linear(x, w, b);
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w0, const OptTensor& b0) {
+    const auto dt = x.scalar_type();
+    const Tensor w = w0.to(dt);
+    ctx->save_for_backward({x, w, w0});
+    ctx->saved_data["bias"] = b0.has_value();
+    return at::linear(x, w, b0 ? OptTensor(b0->to(dt)) : OptTensor());
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
     const Needs n(ctx, {true, true, ctx->saved_data["bias"].toBool()});
-    const Tensor &x = s[0], &w = s[1], &dy = g[0];
-    const int64_t O = w.size(0), I = w.size(1);
+    const Tensor &x = s[0], &w0 = s[2], &dy = g[0];
+    const int64_t O = w0.size(0), I = w0.size(1);
+    const auto out = w0.scalar_type();
     Tensor dx, dw, db;
-    if (n.need[0]) dx = at::matmul(dy, w);
+    // Under create_graph the gradients are themselves differentiated: plain products of the inputs.
+    const bool plain = at::GradMode::is_enabled();
+    if (n.need[0]) dx = at::matmul(dy, plain ? w0.to(x.scalar_type()) : s[1]);
     if (n.need[1] || n.need[2]) {
       const Tensor dy2 = dy.reshape({-1, O});
-      // Under create_graph the gradients are themselves differentiated: plain products.
-      if (n.need[1] && !at::GradMode::is_enabled() && dy.scalar_type() == x.scalar_type() &&
+      if (n.need[1] && !plain && dy.scalar_type() == x.scalar_type() &&
           use_wgrad(x.scalar_type(), dy2.size(0), O, I)) {
-        linear_wgrad(dy2, x.reshape({-1, I}), n.need[2], dw, db);
+        linear_wgrad(dy2, x.reshape({-1, I}), out, n.need[2], dw, db);
       } else {
-        if (n.need[1]) dw = dy2.t().mm(x.reshape({-1, I}));
-        if (n.need[2]) db = dy2.sum(0);
+        if (n.need[1]) dw = dy2.t().mm(x.reshape({-1, I})).to(out);
+        if (n.need[2]) db = dy2.sum(0).to(out);
       }
     }
     return {dx, dw, db};
   }
 };
 
-// F.linear on GPU tensors.  Under autocast the operands are cast as F.linear's are (the same cached
-// weight casts); anything but 16-bit training on plain tensors is F.linear itself.
+// F.linear on GPU tensors.  Under autocast the operands take the types F.linear's would; anything
+// but 16-bit training on plain tensors is F.linear itself.
 Tensor linear(const Tensor& x0, const Tensor& w0, const OptTensor& b0) {
   py::gil_scoped_release nogil;
   auto plain = [](const Tensor& t) { return t.is_cuda() && !t.key_set().has(c10::DispatchKey::Python); };
   if (!at::GradMode::is_enabled() || !w0.requires_grad() || !plain(x0) || !plain(w0) || (b0 && !plain(*b0)) ||
-      x0.dim() < 2 || w0.dim() != 2 || x0.numel() == 0)
+      x0.dim() < 2 || w0.dim() != 2 || x0.numel() == 0 || (b0 && b0->scalar_type() != w0.scalar_type()))
     return at::linear(x0, w0, b0);
-  Tensor x = x0, w = w0;
-  OptTensor b = b0;
-  if (at::autocast::is_autocast_enabled(at::kCUDA)) {
-    const auto dt = at::autocast::get_autocast_dtype(at::kCUDA);
-    x = at::autocast::cached_cast(dt, x, at::kCUDA);
-    w = at::autocast::cached_cast(dt, w, at::kCUDA);
-    if (b) b = at::autocast::cached_cast(dt, *b, at::kCUDA);
-  }
-  const auto dt = x.scalar_type();
-  if (dt != w.scalar_type() || (b && dt != b->scalar_type()) || x.size(-1) != w.size(1) ||
-      !use_wgrad(dt, x.numel() / x.size(-1), w.size(0), w.size(1)))
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  const auto dt = autocast ? at::autocast::get_autocast_dtype(at::kCUDA) : x0.scalar_type();
+  const auto wt = w0.scalar_type();
+  const bool types_ok = autocast ? (wt == at::kFloat || wt == dt) && (x0.scalar_type() == at::kFloat || kernel_dtype(x0.scalar_type()) ||
+                                                                      x0.scalar_type() == at::kHalf)
+                                 : wt == dt;
+  if (!types_ok || x0.size(-1) != w0.size(1) || !use_wgrad(dt, x0.numel() / x0.size(-1), w0.size(0), w0.size(1)))
     return at::linear(x0, w0, b0);
-  return LinearFunction::apply(x, w, b);
+  return LinearFunction::apply(autocast ? at::autocast::cached_cast(dt, x0, at::kCUDA) : x0, w0, b0);
 }
 
 void init(const py::dict& addresses, const py::object& library_error) {

@@ -2,7 +2,8 @@
 //
 //     dW[o,i] = sum_t dy[t,o] x[t,i],     db[o] = sum_t dy[t,o],
 //
-// dy [T,O], x [T,I], both bf16 or both f16, sums in float32, results rounded once to that type.
+// dy [T,O], x [T,I], both bf16 or both f16, sums in float32, results in that type (rounded once) or
+// in float32 (the parameters' type under autocast: no cast afterwards).
 //
 // A model's weight is small and its row count is not (256 x 256 over 16384 rows): a product tiled
 // over the output alone has a handful of tiles, each walking every row (the library's choice for
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(kBlock, 2) void linear_wgrad_kernel(LinearParams p)
 
 // Sum of the splits' partials, four elements per lane; a workgroup's four waves take a quarter of
 // the splits each and meet in LDS (in wave order).  n is the element count (a multiple of 4).
-template <bool F16>
+template <bool F16, bool OUT32>
 __device__ __forceinline__ void reduce_four(const float* part, void* out, long long n, long long blk, int splits,
                                             float4 (&sh)[4][64]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -193,6 +194,10 @@ __device__ __forceinline__ void reduce_four(const float* part, void* out, long l
     for (int k = 1; k < 4; ++k) {
       s.x += sh[k][l].x; s.y += sh[k][l].y; s.z += sh[k][l].z; s.w += sh[k][l].w;
     }
+    if constexpr (OUT32) {
+      *reinterpret_cast<float4*>(static_cast<float*>(out) + e) = s;
+      return;
+    }
     uint2 o;
     if constexpr (F16) {
       typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
@@ -204,13 +209,13 @@ __device__ __forceinline__ void reduce_four(const float* part, void* out, long l
   }
 }
 
-template <bool F16>
+template <bool F16, bool OUT32>
 __global__ __launch_bounds__(kBlock) void linear_reduce_kernel(LinearParams p, int w_blocks) {
   __shared__ float4 sh[4][64];
   if ((int)blockIdx.x < w_blocks)
-    reduce_four<F16>(p.part, p.dw, (long long)p.O * p.I, blockIdx.x, p.splits, sh);
+    reduce_four<F16, OUT32>(p.part, p.dw, (long long)p.O * p.I, blockIdx.x, p.splits, sh);
   else
-    reduce_four<F16>(p.part_b, p.db, p.O, blockIdx.x - w_blocks, p.splits, sh);
+    reduce_four<F16, OUT32>(p.part_b, p.db, p.O, blockIdx.x - w_blocks, p.splits, sh);
 }
 
 // One 128 x 128 tile per CU and split: as many splits as give a workgroup to every CU, of at least
@@ -231,6 +236,7 @@ size_t linear_align(size_t x) { return (x + 255) & ~size_t(255); }
 int linear_check(const dsqg_linear_wgrad_args* a, LinearParams* p) {
   if (!a || a->T < 0 || a->O <= 0 || a->I <= 0 || a->O % 8 != 0 || a->I % 8 != 0) return DSQG_EINVAL;
   if (a->dtype != DSQG_BF16 && a->dtype != DSQG_F16) return DSQG_EINVAL;
+  if (a->out_dtype != a->dtype && a->out_dtype != DSQG_F32) return DSQG_EINVAL;
   if (a->T == 0 || (long long)a->O * a->I >= (1ll << 31)) return DSQG_EUNSUPPORTED;
   *p = LinearParams{};
   p->T = a->T; p->O = a->O; p->I = a->I;
@@ -276,12 +282,10 @@ extern "C" int dsqg_linear_wgrad(const dsqg_linear_wgrad_args* a, dsqg_stream_t 
   const dim3 grid((unsigned)(p.splits * p.to * p.ti));
   const int w_blocks = (int)(((long long)p.O * p.I + 255) / 256);
   const dim3 rgrid((unsigned)(w_blocks + (a->db ? (p.O + 255) / 256 : 0)));
-  if (a->dtype == DSQG_F16) {
-    hipLaunchKernelGGL((linear_wgrad_kernel<true>), grid, dim3(kBlock), 0, st, p);
-    hipLaunchKernelGGL((linear_reduce_kernel<true>), rgrid, dim3(kBlock), 0, st, p, w_blocks);
-  } else {
-    hipLaunchKernelGGL((linear_wgrad_kernel<false>), grid, dim3(kBlock), 0, st, p);
-    hipLaunchKernelGGL((linear_reduce_kernel<false>), rgrid, dim3(kBlock), 0, st, p, w_blocks);
-  }
+  if (a->dtype == DSQG_F16) hipLaunchKernelGGL((linear_wgrad_kernel<true>), grid, dim3(kBlock), 0, st, p);
+  else hipLaunchKernelGGL((linear_wgrad_kernel<false>), grid, dim3(kBlock), 0, st, p);
+  if (a->out_dtype == DSQG_F32) hipLaunchKernelGGL((linear_reduce_kernel<false, true>), rgrid, dim3(kBlock), 0, st, p, w_blocks);
+  else if (a->dtype == DSQG_F16) hipLaunchKernelGGL((linear_reduce_kernel<true, false>), rgrid, dim3(kBlock), 0, st, p, w_blocks);
+  else hipLaunchKernelGGL((linear_reduce_kernel<false, false>), rgrid, dim3(kBlock), 0, st, p, w_blocks);
   return hipGetLastError() == hipSuccess ? DSQG_OK : DSQG_EHIP;
 }

@@ -301,11 +301,12 @@ int dsqg_pool_gate_bwd(const dsqg_pool_gate_bwd_args* args, dsqg_stream_t stream
  * train/train_2048_condU.py:126-130, 244-246): dw[o,i] = sum_t dy[t,o] x[t,i] and, when db is
  * given, db[o] = sum_t dy[t,o].  dy [T,O] and x [T,I] have unit column stride, row strides that are
  * a multiple of 8 elements and 16-byte aligned bases; O and I are multiples of 8, T >= 1; dw [O,I]
- * and db [O] are contiguous and 16-byte aligned.  dtype is F16 or BF16, of all four; sums are
- * fp32 and deterministic, rounded once. */
+ * and db [O] are contiguous and 16-byte aligned.  Sums are fp32 and deterministic, rounded once to
+ * out_dtype. */
 typedef struct {
     int32_t T, O, I;
-    int32_t dtype;             /* DSQG_F16 or DSQG_BF16 */
+    int32_t dtype;             /* DSQG_F16 or DSQG_BF16, of dy and x */
+    int32_t out_dtype;         /* that, or DSQG_F32, of dw and db */
     const void* dy;  int64_t dy_stride;
     const void* x;   int64_t x_stride;
     void* dw;

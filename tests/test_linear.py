@@ -1,8 +1,8 @@
 """Weight and bias gradients of the linear layers: the kernel against float64 at the edges of its
 tiles and row splits, and the layer against nn.Linear through autograd and autocast.
 
-A sum of T products rounded once to the 16-bit type is within half an ulp (2^-11 of the value in
-float16, 2^-8 in bfloat16) plus the float32 sum's rounding, below T 2^-24 of its terms' magnitude.
+A sum of T products rounded once to the output type is within half an ulp (2^-11 of the value in
+float16, 2^-8 in bfloat16, 2^-24 in float32) plus the float32 sum's rounding, below T 2^-24 of its terms' magnitude.
 """
 
 import ctypes
@@ -15,7 +15,7 @@ from torch import nn
 from dwarf_amd import _lib
 from dwarf_amd.modules import Linear
 
-HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
 
 
 def _close(got, dy, x, name):
@@ -36,7 +36,7 @@ def test_kernel_against_float64(gpu_device, T, O, I, pad, dtype):
     x = torch.randn(T, I + pad, generator=g).to(gpu_device, dtype)[:, :I]
     a = _lib.LinearWgradArgs()
     a.T, a.O, a.I = T, O, I
-    a.dtype = _lib.DSQG_F16 if dtype == torch.float16 else _lib.DSQG_BF16
+    a.dtype = a.out_dtype = _lib.DSQG_F16 if dtype == torch.float16 else _lib.DSQG_BF16
     a.dy, a.dy_stride, a.x, a.x_stride = dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0)
     dw = torch.full((O, I), float("nan"), device=gpu_device, dtype=dtype)
     db = torch.full((O,), float("nan"), device=gpu_device, dtype=dtype)
@@ -57,13 +57,13 @@ def test_arguments_are_checked_on_the_host():
     lib = _lib.load()
     n = ctypes.c_size_t(0)
     a = _lib.LinearWgradArgs()
-    a.T, a.O, a.I, a.dtype = 64, 16, 24, _lib.DSQG_BF16
+    a.T, a.O, a.I, a.dtype, a.out_dtype = 64, 16, 24, _lib.DSQG_BF16, _lib.DSQG_BF16
     assert lib.dsqg_linear_wgrad_workspace_size(ctypes.byref(a), ctypes.byref(n)) == _lib.DSQG_OK
     assert lib.dsqg_linear_wgrad(ctypes.byref(a), None) == _lib.DSQG_EINVAL  # no tensors
     a.dy = a.x = a.dw = a.db = 0x10000
     a.dy_stride, a.x_stride = 16, 24
     assert lib.dsqg_linear_wgrad(ctypes.byref(a), None) == _lib.DSQG_EWORKSPACE
-    for field, value in (("O", 12), ("I", 0), ("T", -1), ("dtype", _lib.DSQG_F32), ("dy_stride", 8),
+    for field, value in (("O", 12), ("I", 0), ("T", -1), ("dtype", _lib.DSQG_F32), ("out_dtype", _lib.DSQG_F16), ("dy_stride", 8),
                          ("x_stride", 28), ("x", 0x10008)):
         b = _lib.LinearWgradArgs.from_buffer_copy(a)
         setattr(b, field, value)
@@ -101,9 +101,24 @@ def test_layer_equals_nn_linear(gpu_device, mode, bias, layout):
             assert torch.equal(u, v)
     if mode != "f32":
         dy2, x2 = dy.reshape(-1, 72), x.to(low).reshape(-1, 48)
-        _close(res[1][2].to(low), dy2, x2, "weight")
+        _close(res[1][2], dy2, x2, "weight")  # (float32 under autocast: not rounded to 16 bits)
         if bias:
-            _close(res[1][3].to(low), dy2, x2[:, :0], "bias")
+            _close(res[1][3], dy2, x2[:, :0], "bias")
+
+
+@pytest.mark.gpu
+def test_second_derivatives_under_autocast(gpu_device):
+    ref, lin = _pair(gpu_device, 48, 72, True, torch.float32)
+    x = torch.randn(64, 48, device=gpu_device)
+    res = []
+    for m in (ref, lin):
+        xi = x.clone().requires_grad_(True)
+        with torch.amp.autocast("cuda"):
+            y = m(xi)
+        (gw,) = torch.autograd.grad(y.float().square().sum(), m.weight, create_graph=True)
+        res.append(torch.autograd.grad(gw.float().square().sum(), [xi, m.weight, m.bias]))
+    for u, v in zip(*res):  # both round dy and dw to float16 on the way
+        assert u.dtype == v.dtype and (u - v).norm() <= 2e-3 * u.norm()
 
 
 @pytest.mark.gpu
