@@ -43,11 +43,12 @@ bool bwd_f32_supported(const BwdParams& p, int D, int dtype) {
 //   B8 H8 N512 D32     24.9 / 30.4 / 43.8      B16 H8 N2048 D32   119 / 103 /  97
 //   B8 H8 N2048 D32      60 /   57 /   64      B8 H24 N2048 D32   168 / 147 / 152
 //   B4 H8 N1024 D64    39.3 / 46.5 / 62.7      B8 H6 N2048 D128   233 / 215 / 237
-//   B2 H12 N2048 D64   46.8 / 51.5             B8 H12 N2048 D64   144 / 134 / 133
+//   B2 H12 N2048 D64   46.8 / 51.5             B8 H6 N2048 D128   182 / 180 / 182
+//   B2 H4 N1024 D128   40.1 / 58.0             B4 H8 N2048 D128   119 / 113 / 138
 //   B8 H8 N2048 D96     151 /  139 /  139      B8 H16 N2048 D96   303 / 272 / 261
 static int se_batches(const BwdParams& p, int D) {
   const int ns = p.taps.J - p.taps.W - 1;
-  const int slots = 256 * (D == 128 ? 1 : D == 32 ? 4 : (D > 64 || ns != 11 ? 2 : 3));  // resident workgroups
+  const int slots = 256 * (D == 32 ? 4 : (D > 64 || ns != 11 ? 2 : 3));  // resident workgroups
   int best = 1;
   double best_cost = 0;
   for (int n : {1, 2, 4}) {

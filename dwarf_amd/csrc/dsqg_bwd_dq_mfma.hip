@@ -47,7 +47,7 @@ constexpr int kDqTableStride = 52;
 // DG: the score gain's gradient is requested (its c q.k table in dynamic LDS and the extra row
 // sums are compiled in only then).
 template <int D, bool HAS_SE, int NSC, bool DG>
-__global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 || (HAS_SE && NSC != 11 && D > 32) ? 2 : ((HAS_SE && D > 32) || DG ? 3 : 4)))
+__global__ __launch_bounds__(kBlock, D == 128 ? (HAS_SE ? 2 : 1) : (D > 64 || (HAS_SE && NSC != 11 && D > 32) ? 2 : ((HAS_SE && D > 32) || DG ? 3 : 4)))
 void bwd_dq_mfma_kernel(BwdParams p) {
   using G_ = Geo<D>;
   constexpr int QT = 64;
@@ -84,10 +84,16 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   // tables during the band, then the [query][tap] tables and the staging blocks (34.4 KB), and
   // four fit.  B8 H8 N2048 with 11 long-range taps: 42.1 -> 35.6 us (two batches each; B16 76 ->
   // 62 with four).
-  constexpr bool PACKED = HAS_SE && D == 32;
+  // At D = 128 likewise (96 KB and one workgroup per CU otherwise).
+  constexpr bool PACKED = HAS_SE && (D == 32 || D == 128);
+  // At D = 128 the scale_embed planes have no LDS of their own either (62.6 KB, two workgroups per
+  // CU): staged in the K window before the window rows (for T) and again after the band (for
+  // SE^T dS).  Whole backward of B8 H6 N2048: 215 -> 180 us.  At D = 80 and 96 the same form would fit three workgroups but needs 228 VGPRs, 84 of
+  // them spilled at the 168 that three allow.
+  constexpr bool RESTAGE = HAS_SE && D == 128;
   constexpr int TBL_B = 4 * 16 * TS * 2;               // bf16 elements of the tables
-  static_assert(!PACKED || (WIN * RV <= TBL_B && 4 * 32 * TST <= TBL_B + 4 * 16 * RV - WIN * RV), "phases fit");
-  __shared__ __align__(16) bf16_t sV[PACKED ? TBL_B + 4 * 16 * RV : WIN * RV];  // dense-window V rows
+  constexpr int PH1 = WIN * RV + 4 * 32 * TST, PH2 = TBL_B + 4 * 16 * RV;
+  __shared__ __align__(16) bf16_t sV[PACKED ? (PH1 > PH2 ? PH1 : PH2) : WIN * RV];  // dense-window V rows
   // Wave-private staging block: with scale_embed first the dense-tap table
   // T[i][j] = log2e (bias_j + c q_i.se_j); then the two rounds that turn dq into row layout;
   // then, with scale_embed, the wave's Q rows (read by every wave for dse).
@@ -96,8 +102,10 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   bf16_t* const sKs = PACKED ? sV + TBL_B : sKsst;
   // scale_embed rows as two bf16 planes, hi = bf16(se) and lo = bf16(se - hi): q.se and
   // SE^T dS then carry se to about 2^-17 relative, as the fp32 se of the reference.
-  __shared__ __align__(16) bf16_t sSE[HAS_SE ? SEJ * RV : 8];
-  __shared__ __align__(16) bf16_t sSElo[HAS_SE ? SEJ * RV : 8];
+  static_assert(2 * SEJ <= WIN, "both planes fit the K window");
+  __shared__ __align__(16) bf16_t sSEst[HAS_SE && !RESTAGE ? 2 * SEJ * RV : 8];
+  bf16_t* const sSE = RESTAGE ? sK : sSEst;
+  bf16_t* const sSElo = sSE + SEJ * RV;
   // [query][tap] per wave: u of the long-range taps (pass 1), then dS.  It lives in the V window
   // once the band is done (D >= 64), which keeps the workgroup's LDS small enough for four
   // workgroups per CU (three with scale_embed).
@@ -153,12 +161,12 @@ void bwd_dq_mfma_kernel(BwdParams p) {
     bias_ld = p.pos_bias[jc * p.H + h];
     gain_ld = p.score_gain ? p.score_gain[h * J + jc] : 1.0f;
     SeRows<D> seR;
-    seR.load(p.scale_embed, J, tid);
+    if constexpr (!RESTAGE) seR.load(p.scale_embed, J, tid);
     if (tid < J) {
       sBias2[tid] = bias_ld * kLog2e;
       sGain[tid] = gain_ld;
     }
-    seR.template store<RV>(sSE, sSElo, tid);
+    if constexpr (!RESTAGE) seR.template store<RV>(sSE, sSElo, tid);
   }
 
   float* const sDS = TBL_IN_V ? reinterpret_cast<float*>(sV) : sDSst;
@@ -217,6 +225,8 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   const bool row_ok = n < N;
 
   // ---- Loads (zero outside [0, N)). ----
+  SeRows<D> seR;
+  if constexpr (RESTAGE) seR.load(p.scale_embed, J, opaque(tid));
   // Dense window K and V rows [n0-32, n0+64), staged once per workgroup in LDS.
   uint4 wk[CWIN], wv[CWIN];
 #pragma unroll
@@ -288,7 +298,35 @@ void bwd_dq_mfma_kernel(BwdParams p) {
     sBias2[tid] = bias_ld * kLog2e;
     sGain[tid] = gain_ld;
   }
+  // T[i][j] = log2e (bias_j + c q_i.se_j) of the dense taps: SE Q^T against both planes.
+  [[maybe_unused]] auto se_table = [&]() {
+#pragma unroll
+    for (int jb = 0; jb < 3; ++jb) {
+      if (16 * jb > W) continue;
+      f32x4_t acc = zero4();
+      const bf16_t* sr = sSE + (16 * jb + i) * RV + 8 * g;
+      const bf16_t* srl = sSElo + (16 * jb + i) * RV + 8 * g;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        acc = mfma_16x16x32(as_bf16x8(*reinterpret_cast<const uint4*>(sr + 32 * s)), qB[s], acc);
+        acc = mfma_16x16x32(as_bf16x8(*reinterpret_cast<const uint4*>(srl + 32 * s)), qB[s], acc);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = 16 * jb + 4 * g + r;
+        if (j <= W) sTw[i * TST + j] = fmaf(c2, acc[r], sBias2[j]);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_wave_barrier();
+  };
   if (tk > 0) __syncthreads();  // the previous slice's reads of the windows and tables are done
+  if constexpr (RESTAGE) {
+    seR.template store<RV>(sSE, sSElo, tid);
+    __syncthreads();
+    se_table();
+    __syncthreads();  // every wave has read the planes: the window rows move in
+  }
 #pragma unroll
   for (int u = 0; u < CWIN; ++u) {
     const int ci = tid + u * kBlock;
@@ -313,27 +351,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
       accU[kk] = mfma_16x16x32(as_bf16x8(*reinterpret_cast<const uint4*>(vr + 32 * s)), oB[s], accU[kk]);
     }
   }
-  if constexpr (HAS_SE) {
-#pragma unroll
-    for (int jb = 0; jb < 3; ++jb) {
-      if (16 * jb > W) continue;
-      f32x4_t acc = zero4();
-      const bf16_t* sr = sSE + (16 * jb + i) * RV + 8 * g;
-      const bf16_t* srl = sSElo + (16 * jb + i) * RV + 8 * g;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        acc = mfma_16x16x32(as_bf16x8(*reinterpret_cast<const uint4*>(sr + 32 * s)), qB[s], acc);
-        acc = mfma_16x16x32(as_bf16x8(*reinterpret_cast<const uint4*>(srl + 32 * s)), qB[s], acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = 16 * jb + 4 * g + r;
-        if (j <= W) sTw[i * TST + j] = fmaf(c2, acc[r], sBias2[j]);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
-  }
+  if constexpr (HAS_SE && !RESTAGE) se_table();
 
   // Dense weights and u; D' collects alpha u of every tap of this lane's query column.
   float al[12], uu[12];
@@ -443,6 +461,12 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   __builtin_amdgcn_wave_barrier();
 
   if constexpr (HAS_SE) {
+    if constexpr (RESTAGE) {
+      seR.load(p.scale_embed, J, opaque(tid));
+      __syncthreads();  // every wave's reads of the K window are done: the planes move in
+      seR.template store<RV>(sSE, sSElo, tid);
+      __syncthreads();
+    }
     // SE^T (c dS)^T from this wave's own table rows: dq's scale_embed term.
 #pragma unroll
     for (int jb = 0; jb < 3; ++jb) {
