@@ -42,7 +42,7 @@ bool bwd_f32_supported(const BwdParams& p, int D, int dtype) {
 //   B4 H4 N256 D64     27.8 / 37.1 / 56.6      B4 H8 N2047 D80     76 /  70 /  84
 //   B8 H8 N512 D32     24.9 / 30.4 / 43.8      B16 H8 N2048 D32   119 / 103 /  97
 //   B8 H8 N2048 D32      60 /   57 /   64      B8 H24 N2048 D32   168 / 147 / 152
-//   B4 H8 N1024 D64    39.3 / 46.5 / 62.7      B8 H6 N2048 D128   233 / 215 / 237
+//   B4 H8 N1024 D64    39.3 / 46.5 / 62.7      B8 H12 N2048 D64   144 / 134 / 133
 //   B2 H12 N2048 D64   46.8 / 51.5             B8 H6 N2048 D128   182 / 180 / 182
 //   B2 H4 N1024 D128   40.1 / 58.0             B4 H8 N2048 D128   119 / 113 / 138
 //   B8 H8 N2048 D96     151 /  139 /  139      B8 H16 N2048 D96   303 / 272 / 261
