@@ -260,8 +260,8 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void bwd_dkdv_f32_kernel(B
   for (int u = 0; u < CHW; ++u) {
     const int rr = rf_row<D>(l, u), cc = rf_col<D>(l, u);
     if (m0w + rr < N) {
-      *reinterpret_cast<float4*>(dkb + (m0w + rr) * p.dks.n + cc) = ka[u];
-      *reinterpret_cast<float4*>(dvb + (m0w + rr) * p.dvs.n + cc) = va[u];
+      store4f_stream(dkb + (m0w + rr) * p.dks.n + cc, ka[u]);
+      store4f_stream(dvb + (m0w + rr) * p.dvs.n + cc, va[u]);
     }
   }
 }

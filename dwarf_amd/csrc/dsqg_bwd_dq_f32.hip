@@ -320,8 +320,8 @@ __global__ __launch_bounds__(kBlock, D <= 64 && !(HAS_SE && DG) ? 2 : 1) void bw
   for (int u = 0; u < CHW; ++u) {
     const int rr = rf_row<D>(l, u);
     if (n0w + rr < N)
-      *reinterpret_cast<float4*>(dqb + (n0w + rr) * p.dqs.n + rf_col<D>(l, u)) =
-          make_float4(c * acc[u].x, c * acc[u].y, c * acc[u].z, c * acc[u].w);
+      store4f_stream(dqb + (n0w + rr) * p.dqs.n + rf_col<D>(l, u),
+                     make_float4(c * acc[u].x, c * acc[u].y, c * acc[u].z, c * acc[u].w));
   }
   if (row_ok && g == 0) p.dpre[rowbase + n] = Dp;
 

@@ -636,7 +636,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
       uint4 o;
       o.x = cvt_pk_bf16(xacc[u][0], xacc[u][1]); o.y = cvt_pk_bf16(xacc[u][2], xacc[u][3]);
       o.z = cvt_pk_bf16(xacc[u][4], xacc[u][5]); o.w = cvt_pk_bf16(xacc[u][6], xacc[u][7]);
-      st16(dqb + (n0w + rr) * p.dqs.n + 8 * cc, o);
+      st16_stream(dqb + (n0w + rr) * p.dqs.n + 8 * cc, o);
     }
   }
   if (row_ok && g == 0) p.dpre[rowbase + n] = Dp;

@@ -110,6 +110,8 @@ __device__ __forceinline__ float bload1f(__amdgpu_buffer_rsrc_t r, int elem) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (unsigned)elem * 4u, 0, 0));
 }
 
+__device__ __forceinline__ void store4f_stream(float* p, float4 x) { st16_stream(p, __builtin_bit_cast(uint4, x)); }
+
 __device__ __forceinline__ float dot4f(float4 a, float4 b, float acc) {
   return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.y, b.y, fmaf(a.x, b.x, acc))));
 }

@@ -263,8 +263,8 @@ __global__ __launch_bounds__(kBlock, D <= 64 ? 2 : 1) void fwd_f32_kernel(FwdPar
     const int rr = rf_row<D>(l, u);
     const float inv = sInv[w][rr];
     if (n0w + rr < N)
-      *reinterpret_cast<float4*>(ob + (n0w + rr) * p.os.n + rf_col<D>(l, u)) =
-          make_float4(acc[u].x * inv, acc[u].y * inv, acc[u].z * inv, acc[u].w * inv);
+      store4f_stream(ob + (n0w + rr) * p.os.n + rf_col<D>(l, u),
+                     make_float4(acc[u].x * inv, acc[u].y * inv, acc[u].z * inv, acc[u].w * inv));
   }
 }
 

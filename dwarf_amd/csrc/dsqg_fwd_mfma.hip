@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kBlock, D == 128 ? 1 : (D > 64 ? 3 : (NSC != 11 ? 3
   for (int u = 0; u < CHW; ++u) {
     const int rr = rc_row<D>(l, u), cc = rc_chunk<D>(l, u);
     if (n0w + rr < N && cc < CPR)
-      st16(outb + (n0w + rr) * p.os.n + 8 * cc, *reinterpret_cast<const uint4*>(sSt + rr * RV + 8 * cc));
+      st16_stream(outb + (n0w + rr) * p.os.n + 8 * cc, *reinterpret_cast<const uint4*>(sSt + rr * RV + 8 * cc));
   }
 }
 

@@ -34,6 +34,7 @@
 namespace dsqg {
 namespace {
 
+constexpr int kStream = 2;  // cache policy of the buffer stores: non-temporal (see st16_stream)
 constexpr int kCpl = 4;                     // channels per lane
 constexpr int kPoolCgt = 16;                // channel groups (lanes across channels) per workgroup
 constexpr int kPoolCh = kPoolCgt * kCpl;    // 64 channels per workgroup
@@ -208,8 +209,8 @@ __device__ __forceinline__ void tstore(const TensorRows& t, int r, const float (
   if (t.dt == DSQG_F32) {
     const u32x2 lo = {__float_as_uint(v[0]), __float_as_uint(v[1])};
     const u32x2 hi = {__float_as_uint(v[2]), __float_as_uint(v[3])};
-    __builtin_amdgcn_raw_buffer_store_b64(lo, t.r, t.lane, r * t.rstep, 0);
-    __builtin_amdgcn_raw_buffer_store_b64(hi, t.r, t.lane + 8, r * t.rstep, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(lo, t.r, t.lane, r * t.rstep, kStream);
+    __builtin_amdgcn_raw_buffer_store_b64(hi, t.r, t.lane + 8, r * t.rstep, kStream);
     return;
   }
   u32x2 w;
@@ -220,7 +221,7 @@ __device__ __forceinline__ void tstore(const TensorRows& t, int r, const float (
     w[0] = pack2_f16(v[0], v[1]);
     w[1] = pack2_f16(v[2], v[3]);
   }
-  __builtin_amdgcn_raw_buffer_store_b64(w, t.r, t.lane, r * t.rstep, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(w, t.r, t.lane, r * t.rstep, kStream);
 }
 
 // Total over the 16 row lanes of each of this lane's channels, returned to every lane:
