@@ -131,7 +131,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
                "+s"(p.vs.b), "+s"(p.vs.h), "+s"(p.vs.n), "+s"(p.dos.b), "+s"(p.dos.h), "+s"(p.dos.n)
                : "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.dout), "s"(p.lse), "s"(p.pos_bias), "s"(p.if_gain),
                  "s"(p.alpha_lr));
-  const int lb = xcd_logical_block(blockIdx.x, nblk);
+  const int lb = xcd_logical_block_reversed(blockIdx.x, nblk);
   // Workgroup lb: tile lb % n_chunks of head h of batch group grp ((grp * H + h) * n_chunks + tile).
   const int gh = lb / p.n_chunks, tile = lb - gh * p.n_chunks;
   const int grp = gh / p.H, h = gh - grp * p.H;

@@ -113,6 +113,16 @@ __device__ __forceinline__ int xcd_logical_block(int bid, int nblocks) {
   return xcd < r ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
 }
 
+// The same ranges, each XCD walking its own from the end: a launch that reads what the launch before
+// it read starts with the (b,h) slices that are still in that XCD's L2.  The bf16 dq runs so between
+// the forward and dk/dv (forward + backward of B4 H8 N4096 D64 102.5 -> 100.6 us, B4 H8 N2047 D80
+// 66.2 -> 64.5, B4 H8 N2048 D128 98.5 -> 95.0; where dq itself is bound by arithmetic: no change).
+__device__ __forceinline__ int xcd_logical_block_reversed(int bid, int nblocks) {
+  const int q = nblocks / kNumXcd, r = nblocks % kNumXcd;
+  const int xcd = bid % kNumXcd, slot = bid / kNumXcd;
+  return xcd < r ? xcd * (q + 1) + q - slot : r * (q + 1) + (xcd - r) * q + q - 1 - slot;
+}
+
 // ---------------------------------------------------------------------------------------
 // Launch parameter blocks (passed by value as kernel arguments).
 // ---------------------------------------------------------------------------------------
