@@ -123,3 +123,29 @@ def test_decode_marks_the_rings_changed(gpu_device):
     # A gradient is still refused, by the op.
     with pytest.raises(RuntimeError):
         dwarf_amd.dsqg_decode_step(rows[0].requires_grad_(True), *rows[1:], *rings, pos, pb).float().sum().backward()
+
+
+class _NoGrad(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@gpu
+@pytest.mark.parametrize("call", ["separate", "qkv", "inject"])
+def test_absent_output_gradient_is_zero(gpu_device, call):
+    """A consumer that returns no gradient: the operands' gradients are zeros, not an error."""
+    qkv, pb, se, sg, ig, deltas = _inputs(gpu_device, torch.float32, "plain")
+    if call == "separate":
+        leaves = [t.contiguous().requires_grad_() for t in qkv.view(B, N, 3, H, D).permute(2, 0, 3, 1, 4)]
+        out = dwarf_amd.dsqg_attention(*leaves, pb, se, score_gain=sg, if_gain=ig)
+    else:
+        leaves = [qkv.requires_grad_(), *(d.requires_grad_() for d in deltas if call == "inject")]
+        out = dwarf_amd.dsqg_attention_qkv(qkv, H, pb, se, score_gain=sg, if_gain=ig,
+                                           kv_inject=tuple(deltas) if call == "inject" else None)
+    for g in torch.autograd.grad(_NoGrad.apply(out).sum(), leaves, allow_unused=True):
+        assert g is None or not g.any()
