@@ -88,8 +88,8 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   constexpr bool PACKED = HAS_SE && (D == 32 || D == 128);
   // At D = 128 the scale_embed planes have no LDS of their own either (62.6 KB, two workgroups per
   // CU): staged in the K window before the window rows (for T) and again after the band (for
-  // SE^T dS).  Whole backward of B8 H6 N2048: 215 -> 180 us.  At D = 80 and 96 the same form would fit three workgroups but needs 228 VGPRs, 84 of
-  // them spilled at the 168 that three allow.
+  // SE^T dS).  Whole backward of B8 H6 N2048: 215 -> 180 us.  At D = 80 and 96 the same form would
+  // fit three workgroups but needs 228 VGPRs, 84 of them spilled at the 168 that three allow.
   constexpr bool RESTAGE = HAS_SE && D == 128;
   constexpr int TBL_B = 4 * 16 * TS * 2;               // bf16 elements of the tables
   constexpr int PH1 = WIN * RV + 4 * 32 * TST, PH2 = TBL_B + 4 * 16 * RV;
@@ -108,7 +108,7 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   bf16_t* const sSElo = sSE + SEJ * RV;
   // [query][tap] per wave: u of the long-range taps (pass 1), then dS.  It lives in the V window
   // once the band is done (D >= 64), which keeps the workgroup's LDS small enough for four
-  // workgroups per CU (three with scale_embed).
+  // workgroups per CU (with scale_embed three at D = 64).
   constexpr bool TBL_IN_V = PACKED || WIN * RV * 2 >= 4 * 16 * TS * 4;
   __shared__ __align__(16) float sDSst[TBL_IN_V ? 4 : 4 * 16 * TS];
   // c q.k per (query, tap), for dg only: dynamic LDS, present when score_gain's gradient is

@@ -66,8 +66,8 @@ typedef enum {
 } dsqg_status;
 
 /* Static scratch of dsqg_bwd_noalloc (bytes per device): the backward workspace of the largest
- * call it takes, as dsqg_bwd_workspace_size reports it (e.g. 37 MB for B8 H12 N2048 D64 with
- * dscale_embed, 1.3 MB without). */
+ * call it takes, as dsqg_bwd_workspace_size reports it (e.g. 18 MB for bf16 B8 H12 N2048
+ * D64 and the 44-offset table with dscale_embed, 10 MB without). */
 #define DSQG_NOALLOC_SCRATCH_BYTES (64u << 20)
 
 /* DSQG_F16 is accepted by the pool entry points only. */

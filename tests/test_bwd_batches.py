@@ -17,7 +17,7 @@ from tests.test_parity_gpu import _rand_inputs, compare, gpu_run, oracle_chunked
     (5, 16, 2048, 64, OFFSETS_V3),    # two batches, the last group of one
     (7, 12, 2048, 64, OFFSETS_V3),    # four, the last group of three
     (3, 8, 2048, 80, OFFSETS_J47),    # two workgroups per CU: two batches, the last group of one
-    (5, 8, 1500, 128, OFFSETS_V3),    # one per CU
+    (5, 8, 1500, 128, OFFSETS_V3),    # two batches, the last group of one, rows of a partial tile
 ])
 def test_batch_plans(gpu_device, B, H, N, D, offsets):
     inp = _rand_inputs(B, H, N, D, offsets, torch.bfloat16, seed=B * N + D, gains=False)
