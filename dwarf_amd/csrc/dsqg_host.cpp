@@ -528,6 +528,7 @@ bool ring_load(const Tensor& k, const Tensor& v, const Tensor& k_ring, const Ten
   py::gil_scoped_release nogil;
   const auto dt = k_ring.scalar_type();
   if (!k_ring.is_cuda() || k.dim() != 4 || k_ring.dim() != 4 || v.sizes() != k.sizes() || v_ring.sizes() != k_ring.sizes() ||
+      v_ring.scalar_type() != dt ||
       k.size(0) != k_ring.size(0) || k.size(1) != k_ring.size(1) || k.size(3) != k_ring.size(3) ||
       (dt != at::kFloat && dt != at::kBFloat16 && dt != at::kHalf) || pos.scalar_type() != at::kLong || pos.dim() != 1 ||
       pos.size(0) != k.size(0) || !pos.is_contiguous() || !k_ring.is_contiguous() || !v_ring.is_contiguous() || k.numel() == 0)

@@ -47,6 +47,22 @@ def test_prefill_equals_indexed_writes(gpu_device, offsets, N, dtype, ring, layo
     assert cache.pos.tolist() == [N] * B and cache.k_ring._version > version
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("types", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+def test_rings_of_two_types(gpu_device, types, rows):
+    """Each ring takes its rows in its own type: the kernel has one type for all four tensors, so
+    this is left to the indexed writes."""
+    B, H, D, N = 2, 3, 32, 29
+    cache = DSQGRingCache(B, H, D, (0, 1, 7), device=gpu_device)
+    cache.k_ring, cache.v_ring = (torch.randn(B, H, cache.S, D, device=gpu_device).to(t) for t in types)
+    k, v = _kv(gpu_device, rows, "plain", B, H, N, D)
+    kr, vr = _reference(cache, k, v)
+    cache.prefill(k, v)
+    assert torch.equal(cache.k_ring, kr) and torch.equal(cache.v_ring, vr)
+    assert cache.pos.tolist() == [N] * B
+
+
 def test_arguments_are_checked_on_the_host():
     lib = _lib.load()
     a = _lib.RingLoadArgs()
