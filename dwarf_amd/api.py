@@ -215,7 +215,6 @@ class DSQGRingCache:
         B, H, N, D = k.shape
         state = (self.k_ring, self.v_ring, self.pos)
         if self.k_ring.is_cuda and not ops.traced(k, v, *state) \
-                and not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)) \
                 and self.S == self.k_ring.shape[2] and _lib.host().ring_load(k, v, *state):
             return
         lo = max(0, N - self.S)

@@ -523,7 +523,9 @@ Tensor decode(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor
 }
 
 // Loads k, v [B,H,N,D] into the rings; false (nothing done) where the kernel does not take these
-// tensors as they are: other shapes, types, layouts or devices.
+// tensors as they are: other shapes, types, layouts or devices, and whatever the indexed writes
+// refuse or see more in than the stored values (a ring that records gradients or is an inference
+// tensor outside inference mode, functorch wrappers, tangents, lazy negation).
 bool ring_load(const Tensor& k, const Tensor& v, const Tensor& k_ring, const Tensor& v_ring, const Tensor& pos) {
   py::gil_scoped_release nogil;
   const auto dt = k_ring.scalar_type();
@@ -539,8 +541,13 @@ bool ring_load(const Tensor& k, const Tensor& v, const Tensor& k_ring, const Ten
     for (int i = 0; i < 3; ++i)
       if (t->stride(i) < 0 || t->stride(i) * es % 16 != 0) return false;
   }
+  const bool grad = at::GradMode::is_enabled(), inference = c10::InferenceMode::is_enabled();
   for (const Tensor* t : {&k, &v, &k_ring, &v_ring, &pos})
-    if (t->device() != k_ring.device() || t->key_set().has(c10::DispatchKey::Python)) return false;
+    if (t->device() != k_ring.device() || t->key_set().has(c10::DispatchKey::Python) || !t->has_storage() || t->is_neg() ||
+        (grad && t->requires_grad()) || t->_fw_grad(0).defined())
+      return false;
+  for (const Tensor* r : {&k_ring, &v_ring, &pos})
+    if (r->is_inference() && !inference) return false;
   for (const Tensor* t : {&k, &v, &k_ring, &v_ring})
     if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
   if (k.size(3) * es % 16 != 0 || k.size(0) * k.size(1) > 65535) return false;

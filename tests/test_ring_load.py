@@ -63,6 +63,46 @@ def test_rings_of_two_types(gpu_device, types, rows):
     assert cache.pos.tolist() == [N] * B
 
 
+@pytest.mark.gpu
+def test_left_to_the_indexed_writes(gpu_device):
+    """What the indexed writes refuse stays refused, and rows that are more than their stored values
+    (lazy negation, tangents, vmap's wrappers) load as there."""
+    B, H, D, N = 2, 3, 32, 5
+    make = lambda: DSQGRingCache(B, H, D, (0, 1, 7), device=gpu_device)
+    k, v = _kv(gpu_device, torch.bfloat16, "plain", B, H, N, D)
+    for name in ("k_ring", "v_ring"):
+        cache = make()
+        getattr(cache, name).requires_grad_(True)
+        with pytest.raises(RuntimeError, match="requires grad"):
+            cache.prefill(k, v)
+        with torch.no_grad():
+            cache.prefill(k, v)
+        assert torch.equal(cache.v_ring[:, :, :N], v)
+    with torch.inference_mode():
+        cache = make()
+        cache.prefill(k, v)
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        cache.prefill(k, v)
+    cache = make()
+    cache.prefill(torch._neg_view(k), v)
+    assert torch.equal(cache.k_ring[:, :, :N], -k)
+    cache = make()
+    with torch.autograd.forward_ad.dual_level():
+        cache.prefill(torch.autograd.forward_ad.make_dual(k, 2 * k), v)
+        tangent = torch.autograd.forward_ad.unpack_dual(cache.k_ring).tangent
+        assert torch.equal(tangent[:, :, :N], 2 * k)
+
+    def load(k_ring, v_ring, pos, k, v):
+        cache = make()
+        cache.k_ring, cache.v_ring, cache.pos = k_ring, v_ring, pos
+        cache.prefill(k, v)
+        return cache.k_ring, cache.pos
+
+    c = make()
+    rings, pos = torch.vmap(load)(*(t.unsqueeze(0).clone() for t in (c.k_ring, c.v_ring, c.pos, k, v)))
+    assert torch.equal(rings[0][:, :, :N], k) and pos.tolist() == [[N] * B]
+
+
 def test_arguments_are_checked_on_the_host():
     lib = _lib.load()
     a = _lib.RingLoadArgs()
