@@ -409,18 +409,22 @@ struct AttentionQkvKvFunction : torch::autograd::Function<AttentionQkvKvFunction
 
 // ---- Public attention calls. ---------------------------------------------------------------------------------
 
-void check_shapes(const Tensor& q, const Tensor& k, const Tensor& v, const Params& P, const Table& t) {
-  require(q.dim() == 4, "q must be [B,H,N,HD], got ", shape_str(q.sizes()));
-  const int64_t H = q.size(1), HD = q.size(3), J = t.J;
-  require(k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v must have the same shape");
+// The per-tap and per-head parameters for H heads of HD over the table t (the kernels index them by these).
+void check_params(const Params& P, int64_t H, int64_t HD, const Table& t) {
   auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
     if (x.defined() && x.sizes() != c10::IntArrayRef(s))
       require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
   };
-  expect(P.pb, {J, H}, "pos_bias");
-  expect(P.se, {J, HD}, "scale_embed");
-  expect(P.sg, {H, J}, "score_gain");
+  expect(P.pb, {t.J, H}, "pos_bias");
+  expect(P.se, {t.J, HD}, "scale_embed");
+  expect(P.sg, {H, t.J}, "score_gain");
   expect(P.ig, {H}, "if_gain");
+}
+
+void check_shapes(const Tensor& q, const Tensor& k, const Tensor& v, const Params& P, const Table& t) {
+  require(q.dim() == 4, "q must be [B,H,N,HD], got ", shape_str(q.sizes()));
+  require(k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v must have the same shape");
+  check_params(P, q.size(1), q.size(3), t);
 }
 
 Params float_params(const Tensor& pb, const OptTensor& se, const OptTensor& sg, const OptTensor& ig) {
@@ -452,14 +456,7 @@ Tensor attention_qkv(const Tensor& qkv0, int64_t H, const Tensor& pb, const OptT
   const int64_t E3 = qkv0.size(2);
   require(H > 0 && E3 % (3 * H) == 0, "qkv last dim ", E3, " is not 3 * num_heads * head_dim");
   const std::vector<int64_t> heads{qkv0.size(0), H, qkv0.size(1), E3 / (3 * H)};
-  auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
-    if (x.defined() && x.sizes() != c10::IntArrayRef(s))
-      require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
-  };
-  expect(pb, {t->J, H}, "pos_bias");
-  expect(undef(se), {t->J, heads[3]}, "scale_embed");
-  expect(undef(sg), {H, t->J}, "score_gain");
-  expect(undef(ig), {H}, "if_gain");
+  check_params({pb, undef(se), undef(sg), undef(ig)}, H, heads[3], *t);
   const auto orig = qkv0.scalar_type();
   const auto dt = kernel_dtype(orig) ? orig : at::kBFloat16;
   const Params P = float_params(pb, se, sg, ig);
@@ -481,14 +478,15 @@ Tensor decode(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor
               const OptTensor& ig0, const py::object& offsets) {
   const TablePtr t = make_table(offsets);
   py::gil_scoped_release nogil;
+  require(k_ring.dim() == 4, "k_ring must be [B,H,S,D], got ", shape_str(k_ring.sizes()));
+  check_params({pb0, undef(se0), undef(sg0), undef(ig0)}, k_ring.size(1), k_ring.size(3), *t);
   auto f32 = [](const Tensor& x) { return x.defined() ? x.detach().to(at::kFloat).contiguous() : x; };
   const Tensor q = q0.contiguous(), k = k0.contiguous(), v = v0.contiguous();
   const Tensor pos = pos0.to(at::kLong).contiguous();
   const Tensor pb = f32(pb0), se = f32(undef(se0)), sg = f32(undef(sg0)), ig = f32(undef(ig0));
   const Tensor out = at::empty_like(q);
-  const c10::Device dev = require_gpu({&q, &k, &v, &k_ring, &v_ring, &pos, &pb, &out});
+  const c10::Device dev = require_gpu({&q, &k, &v, &k_ring, &v_ring, &pos, &pb, &se, &sg, &ig, &out});
   const c10::OptionalDeviceGuard guard(dev);
-  require(k_ring.dim() == 4, "k_ring must be [B,H,S,D], got ", shape_str(k_ring.sizes()));
   const int64_t B = k_ring.size(0), H = k_ring.size(1), S = k_ring.size(2), D = k_ring.size(3);
   const auto dt = q.scalar_type();
   require(kernel_dtype(dt) && k.scalar_type() == dt && v.scalar_type() == dt && k_ring.scalar_type() == dt &&

@@ -486,9 +486,15 @@ def decode_step_into(q, k_new, v_new, k_ring, v_ring, pos, pos_bias, scale_embed
     Every tensor must already be contiguous on the GPU and parameters fp32, so the call
     allocates nothing and can be captured in a HIP graph.
     """
-    dev = _require_gpu(q, k_new, v_new, k_ring, v_ring, pos, pos_bias, out)
-    lib = _lib.load()
     B, H, S, D = k_ring.shape
+    J = len(offsets)
+    for name, t, shp in (("pos_bias", pos_bias, (J, H)), ("scale_embed", scale_embed, (J, D)),
+                         ("score_gain", score_gain, (H, J)), ("if_gain", if_gain, (H,))):
+        if t is not None and tuple(t.shape) != shp:
+            raise AssertionError(f"{name} must be {shp}, got {tuple(t.shape)}")
+    dev = _require_gpu(q, k_new, v_new, k_ring, v_ring, pos, pos_bias, scale_embed, score_gain,
+                       if_gain, out)
+    lib = _lib.load()
     code = _DTYPE_CODE.get(q.dtype)
     if code is None or any(t.dtype != q.dtype for t in (k_new, v_new, k_ring, v_ring, out)):
         raise AssertionError("q, k_new, v_new, rings and out must share dtype float32 or bfloat16")

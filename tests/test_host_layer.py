@@ -36,6 +36,41 @@ def test_refuses_cpu_tensors_and_bad_shapes():
         dwarf_amd.dsqg_attention_qkv(torch.zeros(1, 4, 190), 2, pb)
 
 
+BAD_DECODE = [dict(pos_bias=(44, 1)), dict(pos_bias=(43, 2)), dict(scale_embed=(44, 16)), dict(scale_embed=(40, 32)),
+              dict(score_gain=(44, 2)), dict(if_gain=(1,))]
+
+
+@pytest.mark.parametrize("bad", BAD_DECODE, ids=lambda b: "-".join(map(str, *b.items())))
+@pytest.mark.parametrize("path", ["eager", "into"])
+def test_decode_refuses_short_parameters(bad, path):
+    """The kernel indexes the parameters by the ring's head count and dim and the table's length."""
+    row, ring = torch.zeros(1, 2, 32), torch.zeros(1, 2, 1537, 32)
+    pos = torch.zeros(1, dtype=torch.int64)
+    kw = {k: torch.zeros(*s) for k, s in bad.items()}
+    pb = kw.pop("pos_bias", torch.zeros(44, 2))
+    with pytest.raises(AssertionError, match="must be"):
+        if path == "eager":
+            dwarf_amd.dsqg_decode_step(row, row, row, ring, ring, pos, pb, offsets=OFFSETS_V3, **kw)
+        else:
+            ops.decode_step_into(row, row, row, ring, ring, pos, pb, kw.get("scale_embed"), kw.get("score_gain"),
+                                 kw.get("if_gain"), list(OFFSETS_V3), torch.empty_like(row))
+
+
+@gpu
+@pytest.mark.parametrize("name,shape", [("scale_embed", (44, 32)), ("score_gain", (2, 44)), ("if_gain", (2,))])
+@pytest.mark.parametrize("path", ["eager", "into"])
+def test_decode_refuses_cpu_parameters(gpu_device, name, shape, path):
+    row, ring = torch.zeros(1, 2, 32, device=gpu_device), torch.zeros(1, 2, 1537, 32, device=gpu_device)
+    pos, pb = torch.zeros(1, dtype=torch.int64, device=gpu_device), torch.zeros(44, 2, device=gpu_device)
+    kw = {name: torch.zeros(*shape)}
+    with pytest.raises(RuntimeError, match="ROCm GPU"):
+        if path == "eager":
+            dwarf_amd.dsqg_decode_step(row, row, row, ring, ring, pos, pb, offsets=OFFSETS_V3, **kw)
+        else:
+            ops.decode_step_into(row, row, row, ring, ring, pos, pb, kw.get("scale_embed"), kw.get("score_gain"),
+                                 kw.get("if_gain"), list(OFFSETS_V3), torch.empty_like(row))
+
+
 def _inputs(dev, dtype, form):
     g = torch.Generator().manual_seed(3)
     qkv = torch.randn(B, N, 3 * H * D, generator=g).to(dev, dtype)
