@@ -684,37 +684,40 @@ void linear_wgrad(const Tensor& dy0, const Tensor& x0, at::ScalarType out, bool 
   check(api.linear_wgrad(&a, stream_of(dev)), "dsqg_linear_wgrad");
 }
 
-// x in the compute type; w and b in it too, or the float32 parameters autocast would cast: then the
-// casts happen here and their gradients come out of the kernel in float32.
+// x and w in the compute type.  Under autocast w is the cast of the float32 parameter w0 and w0 is
+// there too: its gradient, and b0's, come out of the kernel in float32, and only the cast copy is
+// saved (the parameter may change before the backward, as under nn.Linear).  Under create_graph the
+// gradients are themselves differentiated: plain products of the inputs, the weight's through w.
 struct LinearFunction : torch::autograd::Function<LinearFunction> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w0, const OptTensor& b0) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& w0, const OptTensor& b0) {
     const auto dt = x.scalar_type();
-    const Tensor w = w0.to(dt);
-    ctx->save_for_backward({x, w, w0});
+    ctx->save_for_backward({x, x.requires_grad() ? w : Tensor()});  // (w serves dx alone)
+    ctx->saved_data["type"] = (int64_t)(w0 ? *w0 : w).scalar_type();
+    ctx->saved_data["cast"] = w0.has_value();
     ctx->saved_data["bias"] = b0.has_value();
     return at::linear(x, w, b0 ? OptTensor(b0->to(dt)) : OptTensor());
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
-    const Needs n(ctx, {true, true, ctx->saved_data["bias"].toBool()});
-    const Tensor &x = s[0], &w0 = s[2], &dy = g[0];
-    const int64_t O = w0.size(0), I = w0.size(1);
-    const auto out = w0.scalar_type();
+    const bool cast = ctx->saved_data["cast"].toBool();
+    const Needs n(ctx, {true, true, cast, ctx->saved_data["bias"].toBool()});
+    const Tensor &x = s[0], &w = s[1], &dy = g[0];
+    const int64_t O = dy.size(-1), I = x.size(-1);
+    const auto out = (at::ScalarType)ctx->saved_data["type"].toInt();
+    const bool plain = at::GradMode::is_enabled(), need_dw = n.need[1] || n.need[2];
     Tensor dx, dw, db;
-    // Under create_graph the gradients are themselves differentiated: plain products of the inputs.
-    const bool plain = at::GradMode::is_enabled();
-    if (n.need[0]) dx = at::matmul(dy, plain ? w0.to(x.scalar_type()) : s[1]);
-    if (n.need[1] || n.need[2]) {
+    if (n.need[0]) dx = at::matmul(dy, w);
+    if (need_dw || n.need[3]) {
       const Tensor dy2 = dy.reshape({-1, O});
-      if (n.need[1] && !plain && dy.scalar_type() == x.scalar_type() &&
-          use_wgrad(x.scalar_type(), dy2.size(0), O, I)) {
-        linear_wgrad(dy2, x.reshape({-1, I}), out, n.need[2], dw, db);
+      if (need_dw && !plain && dy.scalar_type() == x.scalar_type() && use_wgrad(x.scalar_type(), dy2.size(0), O, I)) {
+        linear_wgrad(dy2, x.reshape({-1, I}), out, n.need[3], dw, db);
       } else {
-        if (n.need[1]) dw = dy2.t().mm(x.reshape({-1, I})).to(out);
-        if (n.need[2]) db = dy2.sum(0).to(out);
+        if (need_dw) dw = dy2.t().mm(x.reshape({-1, I}));
+        if (n.need[3]) db = dy2.sum(0).to(out);
       }
     }
-    return {dx, dw, db};
+    if (!cast || plain) return {dx, dw, Tensor(), db};
+    return {dx, Tensor(), dw.defined() ? dw.to(out) : dw, db};
   }
 };
 
@@ -734,7 +737,9 @@ Tensor linear(const Tensor& x0, const Tensor& w0, const OptTensor& b0) {
                                  : wt == dt;
   if (!types_ok || x0.size(-1) != w0.size(1) || !use_wgrad(dt, x0.numel() / x0.size(-1), w0.size(0), w0.size(1)))
     return at::linear(x0, w0, b0);
-  return LinearFunction::apply(autocast ? at::autocast::cached_cast(dt, x0, at::kCUDA) : x0, w0, b0);
+  if (!autocast) return LinearFunction::apply(x0, w0, OptTensor(), b0);
+  return LinearFunction::apply(at::autocast::cached_cast(dt, x0, at::kCUDA), at::autocast::cached_cast(dt, w0, at::kCUDA),
+                               wt == dt ? OptTensor() : OptTensor(w0), b0);
 }
 
 void init(const py::dict& addresses, const py::object& library_error) {

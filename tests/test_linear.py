@@ -149,3 +149,48 @@ def test_layer_keeps_nn_linears_contract(gpu_device):
     with torch.autograd.forward_ad.dual_level():
         d = torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x))
         assert torch.autograd.forward_ad.unpack_dual(lin(d)).tangent is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["autocast", "bf16"])
+@pytest.mark.parametrize("x_grad", [True, False])
+def test_weight_changed_before_the_backward(gpu_device, mode, x_grad):
+    """nn.Linear saves what its backward reads: under autocast the cast weight, and no weight where x
+    takes no gradient.  A parameter changed in place in between is accepted exactly where it is there."""
+    pair = _pair(gpu_device, 48, 72, True, torch.float32 if mode == "autocast" else torch.bfloat16)
+    x = torch.randn(64, 48, device=gpu_device).to(torch.float32 if mode == "autocast" else torch.bfloat16)
+    res = []
+    for m in pair:
+        xi = x.clone().requires_grad_(x_grad)
+        with torch.amp.autocast("cuda", enabled=mode == "autocast"):
+            y = m(xi)
+        with torch.no_grad():
+            m.weight.add_(1.0)
+        leaves = [*([xi] if x_grad else []), m.weight, m.bias]
+        try:
+            res.append(torch.autograd.grad(y, leaves, torch.linspace(-1, 1, y.numel(), device=gpu_device).view(y.shape).to(y.dtype)))
+        except RuntimeError as e:
+            res.append("modified by an inplace operation" in str(e))
+    if mode == "bf16" and x_grad:
+        assert res == [True, True]
+        return
+    for u, v in zip(*res):  # (dw and db: float32 sums, rounded to 16 bits by nn.Linear)
+        assert u.dtype == v.dtype and (u - v).float().norm() <= 4e-3 * u.float().norm()
+    if x_grad:
+        assert torch.equal(res[0][0], res[1][0])
+
+
+@pytest.mark.gpu
+def test_second_derivatives_after_a_weight_change(gpu_device):
+    """Under autocast the graph of the gradients reads the weight as it was at the forward."""
+    res = []
+    for m in _pair(gpu_device, 48, 72, True, torch.float32):
+        x = torch.linspace(-1, 1, 64 * 48, device=gpu_device).view(64, 48).requires_grad_(True)
+        with torch.amp.autocast("cuda"):
+            y = m(x)
+        with torch.no_grad():
+            m.weight.mul_(3.0)
+        gx, gw = torch.autograd.grad(y.float().square().sum(), [x, m.weight], create_graph=True)
+        res.append(torch.autograd.grad(gx.square().sum() + gw.square().sum(), [x, m.weight, m.bias]))
+    for u, v in zip(*res):
+        assert u.dtype == v.dtype and (u - v).norm() <= 2e-3 * u.norm()
