@@ -650,7 +650,7 @@ Tensor pool_gate(const Tensor& x, const Tensor& g) {
 // 16384 x 256 x 256 17 / 122, 16384 x 768 x 768 50 / 124, 16384 x 3072 x 768 157 / 224,
 // 65536 x 2304 x 768 430 / 609; 65536 x 3072 x 768 578 / 548.
 bool use_wgrad(at::ScalarType dt, int64_t T, int64_t O, int64_t I) {
-  if ((dt != at::kHalf && dt != at::kBFloat16) || T < 1 || O % 8 != 0 || I % 8 != 0) return false;
+  if ((dt != at::kHalf && dt != at::kBFloat16) || T < 1 || O < 1 || O % 8 != 0 || I % 8 != 0) return false;
   if ((T + 128) * std::max(O, I) * 2 >= (1ll << 31)) return false;
   return O * I <= (1ll << 21) || (O * I <= 3072 * 768 && T <= 16384);
 }

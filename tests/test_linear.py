@@ -194,3 +194,12 @@ def test_second_derivatives_after_a_weight_change(gpu_device):
         res.append(torch.autograd.grad(gx.square().sum() + gw.square().sum(), [x, m.weight, m.bias]))
     for u, v in zip(*res):
         assert u.dtype == v.dtype and (u - v).norm() <= 2e-3 * u.norm()
+
+
+@pytest.mark.gpu
+def test_layer_without_outputs(gpu_device):
+    for m in _pair(gpu_device, 48, 0, True, torch.bfloat16):
+        x = torch.randn(64, 48, device=gpu_device).bfloat16().requires_grad_(True)
+        y = m(x)
+        y.sum().backward()
+        assert y.shape == (64, 0) and m.weight.grad.shape == (0, 48) and not x.grad.any()
