@@ -345,7 +345,7 @@ Injected inject(const Tensor& qkv, const Tensor& kd, const Tensor& vd, int64_t H
   if (qkv.numel() == 0 || HD % 8 != 0 || E * qkv.element_size() % 16 != 0 || kd.scalar_type() != qkv.scalar_type() ||
       vd.scalar_type() != qkv.scalar_type() || !kd.is_cuda() || !vd.is_cuda() || !qkv.is_cuda() ||
       kd.device() != qkv.device() || vd.device() != qkv.device() || (cast && qkv.scalar_type() != at::kHalf) ||
-      !aligned(qkv) || !aligned(kd) || !aligned(vd)) {
+      kd.is_neg() || vd.is_neg() || !aligned(qkv) || !aligned(kd) || !aligned(vd)) {
     const Tensor x = qkv.to(dt);
     return {head_view(x, H, 0), head_view(x, H, 1) + kd.to(dt), head_view(x, H, 2) + vd.to(dt)};
   }
@@ -666,7 +666,7 @@ Tensor wgrad_rows(const Tensor& t) {
 void linear_wgrad(const Tensor& dy0, const Tensor& x0, at::ScalarType out, bool need_db, Tensor& dw, Tensor& db) {
   const c10::Device dev = require_gpu({&dy0, &x0});
   const c10::OptionalDeviceGuard guard(dev);
-  const Tensor dy = wgrad_rows(dy0), x = wgrad_rows(x0);
+  const Tensor dy = wgrad_rows(dy0.resolve_neg()), x = wgrad_rows(x0);
   dw = at::empty({dy.size(1), x.size(1)}, x.options().dtype(out));
   if (need_db) db = at::empty({dy.size(1)}, x.options().dtype(out));
   dsqg_linear_wgrad_args a = {};
@@ -725,7 +725,9 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
 // but 16-bit training on plain tensors is F.linear itself.
 Tensor linear(const Tensor& x0, const Tensor& w0, const OptTensor& b0) {
   py::gil_scoped_release nogil;
-  auto plain = [](const Tensor& t) { return t.is_cuda() && !t.key_set().has(c10::DispatchKey::Python); };
+  auto plain = [](const Tensor& t) {
+    return t.is_cuda() && t.layout() == at::kStrided && !t.is_neg() && !t.key_set().has(c10::DispatchKey::Python);
+  };
   if (!at::GradMode::is_enabled() || !w0.requires_grad() || !plain(x0) || !plain(w0) || (b0 && !plain(*b0)) ||
       x0.dim() < 2 || w0.dim() != 2 || x0.numel() == 0 || (b0 && b0->scalar_type() != w0.scalar_type()))
     return at::linear(x0, w0, b0);

@@ -46,6 +46,17 @@ def test_equals_casts_and_adds(gpu_device, D, dtype, delta, layout):
         assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v)
 
 
+@pytest.mark.gpu
+def test_lazily_negated_deltas(gpu_device):
+    torch.manual_seed(0)
+    qkv = torch.randn(B, N, 3 * H * 32, device=gpu_device).bfloat16()
+    kd, vd = _deltas(gpu_device, torch.bfloat16, "tokens", 32)
+    pb = torch.randn(len(OFFSETS_V3), H, device=gpu_device)
+    out = [dwarf_amd.dsqg_attention_qkv(qkv, H, pb, kv_inject=d)
+           for d in ((torch._neg_view(kd), torch._neg_view(vd)), (-kd, -vd))]
+    assert torch.equal(*out)
+
+
 def test_arguments_are_checked_on_the_host():
     lib = _lib.load()
     a = _lib.KvInjectArgs()

@@ -203,3 +203,13 @@ def test_layer_without_outputs(gpu_device):
         y = m(x)
         y.sum().backward()
         assert y.shape == (64, 0) and m.weight.grad.shape == (0, 48) and not x.grad.any()
+
+
+@pytest.mark.gpu
+def test_lazily_negated_operands(gpu_device):
+    ref, lin = _pair(gpu_device, 48, 72, True, torch.bfloat16)
+    x = torch.randn(64, 48, device=gpu_device).bfloat16()
+    dy = torch.randn(64, 72, device=gpu_device).bfloat16()
+    for xi, g in ((torch._neg_view(x), dy), (x, torch._neg_view(dy))):
+        res = [torch.autograd.grad(m(xi), m.weight, g)[0].float() for m in (ref, lin)]
+        assert (res[0] - res[1]).norm() <= 4e-3 * res[0].norm()
