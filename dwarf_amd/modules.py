@@ -51,11 +51,18 @@ class Linear(nn.Linear):
     alone and a column sum.  Parameters, hooks, autocast and results' types are nn.Linear's."""
 
     def forward(self, x: Tensor) -> Tensor:
-        if not x.is_cuda or ops.traced(x, self.weight) or fwAD._current_level >= 0 \
-                or has_torch_function((x, self.weight)) \
-                or torch._C._functorch.peek_interpreter_stack() is not None:
+        if torch.jit.is_scripting():
             return F.linear(x, self.weight, self.bias)
-        return _lib.host().linear(x, self.weight, self.bias)
+        else:  # (not compiled by torch.jit.script)
+            return _linear(x, self.weight, self.bias)
+
+
+def _linear(x: Tensor, weight: Tensor, bias: Optional[Tensor]) -> Tensor:
+    # (First of all proxies and tensor subclasses: torch.fx traces F.linear.)
+    if has_torch_function((x, weight)) or not x.is_cuda or ops.traced(x, weight) \
+            or fwAD._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+        return F.linear(x, weight, bias)
+    return _lib.host().linear(x, weight, bias)
 
 
 def _log_linear_bias(offsets: Sequence[int], num_heads: int) -> Tensor:

@@ -13,7 +13,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from dwarf_amd import _lib
-from dwarf_amd.modules import Linear
+from dwarf_amd.modules import FFN, Linear
 
 HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
 
@@ -213,3 +213,19 @@ def test_lazily_negated_operands(gpu_device):
     for xi, g in ((torch._neg_view(x), dy), (x, torch._neg_view(dy))):
         res = [torch.autograd.grad(m(xi), m.weight, g)[0].float() for m in (ref, lin)]
         assert (res[0] - res[1]).norm() <= 4e-3 * res[0].norm()
+
+
+@pytest.mark.parametrize("trace", [torch.jit.script, torch.fx.symbolic_trace, "export", "compile"],
+                         ids=["script", "fx", "export", "compile"])
+def test_layers_can_be_traced(trace):
+    """What takes a model of nn.Linear layers takes these (here without a GPU)."""
+    torch.manual_seed(0)
+    ffn = FFN(32, 64).eval()
+    x = torch.randn(3, 32)
+    if trace == "export":
+        run = torch.export.export(ffn, (x,)).module()
+    elif trace == "compile":
+        run = torch.compile(ffn, backend="eager", fullgraph=True)
+    else:
+        run = trace(ffn)
+    assert torch.equal(run(x), ffn(x))
