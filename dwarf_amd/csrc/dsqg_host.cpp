@@ -684,18 +684,33 @@ void linear_wgrad(const Tensor& dy0, const Tensor& x0, at::ScalarType out, bool 
   check(api.linear_wgrad(&a, stream_of(dev)), "dsqg_linear_wgrad");
 }
 
-// x and w in the compute type.  Under autocast w is the cast of the float32 parameter w0 and w0 is
-// there too: its gradient, and b0's, come out of the kernel in float32, and only the cast copy is
-// saved (the parameter may change before the backward, as under nn.Linear).  Under create_graph the
-// gradients are themselves differentiated: plain products of the inputs, the weight's through w.
+// w with the history of a cast of w0.
+struct CastOf : torch::autograd::Function<CastOf> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& w0, const Tensor& w) {
+    ctx->saved_data["type"] = (int64_t)w0.scalar_type();
+    return w;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+    return {g[0].to((at::ScalarType)ctx->saved_data["type"].toInt()), Tensor()};
+  }
+};
+
+// x in the compute type; w in it too, or the float32 leaf parameter that autocast would cast: the
+// cast happens here, its gradient and b0's come out of the kernel in float32, and only the copy is
+// saved (the parameter may change before the backward, as under nn.Linear).  A weight with a history
+// of its own comes as its cast w and, for the float32 gradient, as w0.  (A cast recorded for every
+// weight costs the block of eight layers 100 us of host time a step.)  Under create_graph the
+// gradients are themselves differentiated: plain products of the inputs, the weight's through its cast.
 struct LinearFunction : torch::autograd::Function<LinearFunction> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& w0, const OptTensor& b0) {
     const auto dt = x.scalar_type();
-    ctx->save_for_backward({x, x.requires_grad() ? w : Tensor()});  // (w serves dx alone)
+    const Tensor wc = w.to(dt);
+    ctx->save_for_backward({x, x.requires_grad() ? wc : Tensor()});  // (the weight serves dx alone)
     ctx->saved_data["type"] = (int64_t)(w0 ? *w0 : w).scalar_type();
     ctx->saved_data["cast"] = w0.has_value();
+    if (w.scalar_type() != dt) ctx->saved_data["leaf"] = w;
     ctx->saved_data["bias"] = b0.has_value();
-    return at::linear(x, w, b0 ? OptTensor(b0->to(dt)) : OptTensor());
+    return at::linear(x, wc, b0 ? OptTensor(b0->to(dt)) : OptTensor());
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
@@ -706,7 +721,10 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
     const auto out = (at::ScalarType)ctx->saved_data["type"].toInt();
     const bool plain = at::GradMode::is_enabled(), need_dw = n.need[1] || n.need[2];
     Tensor dx, dw, db;
-    if (n.need[0]) dx = at::matmul(dy, w);
+    if (n.need[0]) {
+      const auto leaf = ctx->saved_data.find("leaf");
+      dx = at::matmul(dy, plain && leaf != ctx->saved_data.end() ? CastOf::apply(leaf->second.toTensor(), w) : w);
+    }
     if (need_dw || n.need[3]) {
       const Tensor dy2 = dy.reshape({-1, O});
       if (need_dw && !plain && dy.scalar_type() == x.scalar_type() && use_wgrad(x.scalar_type(), dy2.size(0), O, I)) {
@@ -716,8 +734,9 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
         if (n.need[3]) db = dy2.sum(0).to(out);
       }
     }
-    if (!cast || plain) return {dx, dw, Tensor(), db};
-    return {dx, Tensor(), dw.defined() ? dw.to(out) : dw, db};
+    if (cast && plain) return {dx, dw, Tensor(), db};
+    if (dw.defined()) dw = dw.to(out);
+    return cast ? variable_list{dx, Tensor(), dw, db} : variable_list{dx, dw, Tensor(), db};
   }
 };
 
@@ -739,9 +758,9 @@ Tensor linear(const Tensor& x0, const Tensor& w0, const OptTensor& b0) {
                                  : wt == dt;
   if (!types_ok || x0.size(-1) != w0.size(1) || !use_wgrad(dt, x0.numel() / x0.size(-1), w0.size(0), w0.size(1)))
     return at::linear(x0, w0, b0);
-  if (!autocast) return LinearFunction::apply(x0, w0, OptTensor(), b0);
-  return LinearFunction::apply(at::autocast::cached_cast(dt, x0, at::kCUDA), at::autocast::cached_cast(dt, w0, at::kCUDA),
-                               wt == dt ? OptTensor() : OptTensor(w0), b0);
+  const Tensor x = autocast ? at::autocast::cached_cast(dt, x0, at::kCUDA) : x0;
+  if (wt == dt || w0.is_leaf()) return LinearFunction::apply(x, w0, OptTensor(), b0);
+  return LinearFunction::apply(x, w0.to(dt), OptTensor(w0), b0);
 }
 
 void init(const py::dict& addresses, const py::object& library_error) {

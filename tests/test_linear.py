@@ -181,17 +181,23 @@ def test_weight_changed_before_the_backward(gpu_device, mode, x_grad):
 
 
 @pytest.mark.gpu
-def test_second_derivatives_after_a_weight_change(gpu_device):
-    """Under autocast the graph of the gradients reads the weight as it was at the forward."""
+@pytest.mark.parametrize("leaf", [True, False])
+def test_second_derivatives_after_a_weight_change(gpu_device, leaf):
+    """Under autocast the graph of the gradients reads the weight as it was at the forward, also where
+    it has a history of its own (weight normalisation)."""
     res = []
     for m in _pair(gpu_device, 48, 72, True, torch.float32):
+        if not leaf:
+            torch.nn.utils.parametrizations.weight_norm(m)
         x = torch.linspace(-1, 1, 64 * 48, device=gpu_device).view(64, 48).requires_grad_(True)
         with torch.amp.autocast("cuda"):
             y = m(x)
-        with torch.no_grad():
-            m.weight.mul_(3.0)
-        gx, gw = torch.autograd.grad(y.float().square().sum(), [x, m.weight], create_graph=True)
-        res.append(torch.autograd.grad(gx.square().sum() + gw.square().sum(), [x, m.weight, m.bias]))
+        params = list(m.parameters())
+        if leaf:
+            with torch.no_grad():
+                m.weight.mul_(3.0)
+        grads = torch.autograd.grad(y.float().square().mean(), [x, *params], create_graph=True)
+        res.append(torch.autograd.grad(sum(g.square().sum() for g in grads), [x, *params]))
     for u, v in zip(*res):
         assert u.dtype == v.dtype and (u - v).norm() <= 2e-3 * u.norm()
 
