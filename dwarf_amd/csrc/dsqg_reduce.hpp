@@ -62,12 +62,20 @@ __device__ __forceinline__ void reduce_params_wave(const ReduceParams& r, int t,
 
 // dscale_embed: workgroup blk sums the partials of 32 consecutive elements of [J*D].  A thread
 // takes four of them (16 bytes; eight lanes read 128 contiguous bytes) of every 32nd partial row,
-// eight rows in flight, and the 32 row sums of an element meet in LDS in order.  lds: 32 x 32
-// floats.  At the start of the dk/dv grid these few workgroups finish long before its tiles do; as
-// a launch of its own between dq and dk/dv (a first stage of 256 slices) the sum cost 5 us.
+// eight rows in flight, and the 32 row sums of an element meet in LDS.  Eight rows are added as a
+// tree, sixteen such sums in turn, those in turn again, and the row sums as a tree: rounding grows
+// with the levels and not with the rows (rms, relative, of unit normals: 3072 partials 1.0e-7, 65536
+// 1.4e-7; one chain per thread and one over the rows 2.1e-7 and 9.0e-7).  lds: 32 x 32 floats.  At
+// the start of the dk/dv grid these few workgroups finish long before its tiles do; as a launch of
+// its own between dq and dk/dv (a first stage of 256 slices) the sum cost 5 us.
 constexpr int kSeGroup = 32;
 
+__device__ __forceinline__ float4 add4f(float4 a, float4 b) {
+  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
 __device__ __forceinline__ void reduce_se_block(const ReduceParams& r, int blk, int tid, float* lds) {
+  constexpr int kRowLanes = kBlock / 8;
   const int JD = r.J * r.D;  // a multiple of 16
   const int c = 4 * (tid & 7), row = tid >> 3;
   const int e = blk * kSeGroup + c;
@@ -75,19 +83,36 @@ __device__ __forceinline__ void reduce_se_block(const ReduceParams& r, int blk, 
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   if (e < JD) {
     const float* src = r.part_se + e;
-#pragma unroll 8
-    for (int k = row; k < rows; k += kBlock / 8) {
-      const float4 x = *reinterpret_cast<const float4*>(src + (long long)k * JD);
-      acc.x += x.x; acc.y += x.y; acc.z += x.z; acc.w += x.w;
+    float4 run = acc;
+    int n = 0;
+    for (int k = row; k < rows; k += 8 * kRowLanes) {
+      float4 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int ku = k + u * kRowLanes;
+        x[u] = *reinterpret_cast<const float4*>(src + (long long)(ku < rows ? ku : k) * JD);
+        if (ku >= rows) x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+      run = add4f(run, add4f(add4f(add4f(x[0], x[1]), add4f(x[2], x[3])), add4f(add4f(x[4], x[5]), add4f(x[6], x[7]))));
+      if (++n == 16) {
+        acc = add4f(acc, run);
+        run = make_float4(0.f, 0.f, 0.f, 0.f);
+        n = 0;
+      }
     }
+    acc = add4f(acc, run);
   }
   *reinterpret_cast<float4*>(lds + row * kSeGroup + c) = acc;
   __syncthreads();
   if (tid < kSeGroup && blk * kSeGroup + tid < JD) {
-    float s = 0.f;
+    float s[kRowLanes];
 #pragma unroll
-    for (int k = 0; k < kBlock / 8; ++k) s += lds[k * kSeGroup + tid];
-    r.dscale_embed[blk * kSeGroup + tid] = s;
+    for (int k = 0; k < kRowLanes; ++k) s[k] = lds[k * kSeGroup + tid];
+#pragma unroll
+    for (int w = kRowLanes / 2; w > 0; w >>= 1)
+#pragma unroll
+      for (int k = 0; k < w; ++k) s[k] += s[k + w];
+    r.dscale_embed[blk * kSeGroup + tid] = s[0];
   }
 }
 
