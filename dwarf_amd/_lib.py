@@ -16,7 +16,7 @@ PKG_DIR = Path(__file__).resolve().parent
 LIB_PATH = Path(os.environ.get("DSQG_HIP_LIB", PKG_DIR / "libdsqg_hip.so"))
 
 MAX_OFFSETS = 64
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 DSQG_OK, DSQG_EINVAL, DSQG_EUNSUPPORTED, DSQG_EHIP, DSQG_EWORKSPACE = 0, 1, 2, 3, 4
 DSQG_ETOOLARGE = 5
@@ -164,20 +164,22 @@ def load() -> ctypes.CDLL:
             f"{LIB_PATH} is missing: build it with `python -m dwarf_amd.build` "
             "(there is no CPU fallback)")
     lib = ctypes.CDLL(str(LIB_PATH))
+    # (The version first: a library of another one need not have every symbol.)
+    ver = lib.dsqg_abi_version() if hasattr(lib, "dsqg_abi_version") else None
+    if ver != ABI_VERSION:
+        raise DSQGLibraryError(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}: build it "
+                               "with `python -m dwarf_amd.build`")
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    ver = lib.dsqg_abi_version()
-    if ver != ABI_VERSION:
-        raise DSQGLibraryError(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}")
     _LIB = lib
     return lib
 
 
 def host():
     """The native host layer (_dsqg_host.so) bound to the library of ``load()``; raise if it is
-    missing."""
+    missing or was compiled against another version of the argument blocks."""
     global _HOST
     if _HOST is not None:
         return _HOST
@@ -188,6 +190,11 @@ def host():
         raise DSQGLibraryError(
             f"the native host layer {PKG_DIR / '_dsqg_host.so'} does not load ({e}): build it with "
             "`python -m dwarf_amd.build`") from e
+    ver = getattr(mod, "abi_version", None)
+    if ver != ABI_VERSION:
+        raise DSQGLibraryError(
+            f"the native host layer {PKG_DIR / '_dsqg_host.so'} has ABI version {ver}, expected "
+            f"{ABI_VERSION}: build it with `python -m dwarf_amd.build`")
     mod.init({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES},
              DSQGLibraryError)
     _HOST = mod

@@ -786,6 +786,7 @@ void init(const py::dict& addresses, const py::object& library_error) {
 
 PYBIND11_MODULE(_dsqg_host, m) {
   m.doc() = "Native host layer of dwarf_amd's eager public functions.";
+  m.attr("abi_version") = DSQG_ABI_VERSION;  // of the argument blocks compiled in here
   m.def("init", &init);
   m.def("attention", &attention);
   m.def("attention_qkv", &attention_qkv);

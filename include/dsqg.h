@@ -47,7 +47,7 @@
 extern "C" {
 #endif
 
-#define DSQG_ABI_VERSION 3
+#define DSQG_ABI_VERSION 4
 #define DSQG_MAX_OFFSETS 64
 
 /* Same type as hipStream_t; NULL is the null stream. */

@@ -316,3 +316,31 @@ def test_bf16_row_span_limit(lib):
         setattr(f, name + "_stride", st)
     f.pos_bias = 0x10000
     assert lib.dsqg_fwd(ctypes.byref(f), None) == _lib.DSQG_EUNSUPPORTED   # refused before a launch
+
+
+@pytest.mark.parametrize("source", ["int dsqg_abi_version(void) { return 3; }", "int other(void) { return 0; }"],
+                         ids=["version", "no-version"])
+def test_library_of_another_version_is_refused(tmp_path, monkeypatch, source):
+    """A library that lacks this version's symbols is refused by its version, not by a missing name."""
+    from dwarf_amd import _lib
+    src, so = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(source + "\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", so)
+    monkeypatch.setattr(_lib, "_LIB", None)
+    with pytest.raises(_lib.DSQGLibraryError, match="ABI version"):
+        _lib.load()
+
+
+@pytest.mark.parametrize("version", [{}, {"abi_version": 3}])
+def test_host_layer_of_another_version_is_refused(lib, monkeypatch, version):
+    import types
+    import dwarf_amd
+    from dwarf_amd import _lib
+    old = types.ModuleType("dwarf_amd._dsqg_host")
+    vars(old).update(version, init=lambda *a: None)
+    monkeypatch.setitem(__import__("sys").modules, "dwarf_amd._dsqg_host", old)
+    monkeypatch.setattr(dwarf_amd, "_dsqg_host", old, raising=False)
+    monkeypatch.setattr(_lib, "_HOST", None)
+    with pytest.raises(_lib.DSQGLibraryError, match="host layer.*ABI version"):
+        _lib.host()
