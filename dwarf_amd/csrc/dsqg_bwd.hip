@@ -38,17 +38,27 @@ bool bwd_f32_supported(const BwdParams& p, int D, int dtype) {
 
 // Batches a workgroup of the bf16 scale_embed dq takes (bwd_plan): the choice of 1, 2 and 4 whose
 // rounds of resident workgroups times batches cost least, counting a partial's store and re-read
-// as 0.6 of a tile (fitted to both directions below).  Whole backward, us, at 1 / 2 / 4 batches:
-//   B4 H4 N256 D64     27.8 / 37.1 / 56.6      B4 H8 N2047 D80     76 /  70 /  84
-//   B8 H8 N512 D32     24.9 / 30.4 / 43.8      B16 H8 N2048 D32   119 / 103 /  97
-//   B8 H8 N2048 D32      60 /   57 /   64      B8 H24 N2048 D32   168 / 147 / 152
-//   B4 H8 N1024 D64    39.3 / 46.5 / 62.7      B8 H12 N2048 D64   144 / 134 / 133
-//   B2 H12 N2048 D64   46.8 / 51.5             B8 H6 N2048 D128   182 / 180 / 182
-//   B2 H4 N1024 D128   40.1 / 58.0             B4 H8 N2048 D128   119 / 113 / 138
-//   B8 H8 N2048 D96     151 /  139 /  139      B8 H16 N2048 D96   303 / 272 / 261
-static int se_batches(const BwdParams& p, int D) {
-  const int ns = p.taps.J - p.taps.W - 1;
-  const int slots = 256 * (D == 32 ? 4 : (D > 64 || ns != 11 ? 2 : 3));  // resident workgroups
+// as 0.6 of a tile.  Whole backward, us, at 1 / 2 / 4 batches, 11 long-range taps, without and with
+// the score gain's gradient (fewer workgroups per CU, so other rounds):
+//   B4 H4 N256 D64     22.5 / 32.1 / 51.5      23.6 / 33.9 / 55.1
+//   B8 H8 N512 D32     21.5 / 26.8 / 39.6      23.0 / 28.3 / 42.3
+//   B8 H8 N2048 D32    49.3 / 47.3 / 55.6      60.4 / 60.7 / 59.9
+//   B16 H8 N2048 D32   86.3 / 82.9 / 81.1     101.5 / 94.7 / 102.5
+//   B4 H8 N1024 D64    29.4 / 35.5 / 54.5      30.1 / 37.1 / 57.9
+//   B2 H12 N2048 D64   34.2 / 42.0             45.2 / 46.5
+//   B4 H8 N2048 D64    50.9 / 48.3 / 62.4      53.5 / 49.1 / 65.2
+//   B8 H12 N2048 D64    113 / 108 / 105         139 / 130 / 138
+//   B4 H8 N4096 D64    80.3 / 81.4 / 83.6      96.8 / 90.7 / 88.5
+//   B4 H8 N2047 D80    63.5 / 61.5 / 76.8      90.2 / 83.5 / 80.8
+//   B8 H8 N2048 D96     123 / 114 / 110         174 / 161 / 155
+//   B2 H4 N1024 D128   36.7 / 54.0             37.9 / 57.1
+//   B4 H8 N2048 D128    108 / 104 / 130         116 / 110 / 137
+//   B8 H6 N2048 D128    156 / 161 / 168         164 / 170 / 180
+// It takes the fastest, or one within 5 %, of each but the last (four: 8 and 10 % over one).  With
+// one count for every form instead it took 2 at B4 H8 N2047 D80 and 4 at B8 H12 N2048 D64 with the
+// gain's gradient, and with 14 taps 2 at B2 H12 N2048 D64 without it (45 us; one batch: 36).
+static int se_batches(const BwdParams& p, int D, bool dg) {
+  const int slots = 256 * bwd_dq_se_resident(D, p.taps.J - p.taps.W - 1, dg);
   int best = 1;
   double best_cost = 0;
   for (int n : {1, 2, 4}) {
@@ -61,7 +71,7 @@ static int se_batches(const BwdParams& p, int D) {
   return best;
 }
 
-void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool compact) {
+void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool dg, bool compact) {
   const bool mfma = bwd_mfma_supported(p, D, dtype);
   const bool tile64 = mfma || bwd_f32_supported(p, D, dtype);
   const int QPB = tile64 ? 64 : kBlock / lanes_per_row(D);  // dq rows per tile
@@ -79,7 +89,7 @@ void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool compact) {
   // dse sums over every b and h, dbias / dg / da over b, so a partial may span batches.
   p.tiles_per_block = 1;
   p.n_chunks = p.n_tiles;
-  p.batches_per_block = !(mfma && se) ? 1 : compact ? (p.B < 4 ? (p.B > 0 ? p.B : 1) : 4) : se_batches(p, D);
+  p.batches_per_block = !(mfma && se) ? 1 : compact ? (p.B < 4 ? (p.B > 0 ? p.B : 1) : 4) : se_batches(p, D, dg);
   p.n_bgroups = (p.B + p.batches_per_block - 1) / p.batches_per_block;
 }
 

@@ -684,6 +684,15 @@ void bwd_dq_mfma_kernel(BwdParams p) {
   }
 }
 
+// From the forms' LDS, with DG's dynamic 13 KB, of a CU's 160 KB: 34.4 + 13.3 KB at D = 32, 51.8 + 13.3
+// at D = 64, 73.9 + 13.3 at D = 80 and 96, 62.6 + 13.3 at D = 128; and from their registers where
+// those allow fewer (D = 64 and a generic table: two; D = 128: two).
+int bwd_dq_se_resident(int D, int ns, bool dg) {
+  if (D == 32) return dg ? 3 : 4;
+  if (D == 64) return dg || (ns != 11 && ns != 13 && ns != 14) ? 2 : 3;
+  return D == 128 || !dg ? 2 : 1;
+}
+
 template <int D, bool HAS_SE>
 static void launch_dq_mfma_ns(const BwdParams& p, unsigned nb, hipStream_t st) {
   if (p.part_gain) {  // the score gain's gradient, with its dg table in dynamic LDS

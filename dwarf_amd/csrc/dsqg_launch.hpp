@@ -24,12 +24,14 @@ hipError_t launch_bwd_dq_f32(const BwdParams& p, int D, unsigned nblocks, hipStr
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
 
 // Tiling of the backward for these sizes and kernel choice; fills n_tiles / tiles_per_block /
-// n_chunks / n_tiles_kv (se: scale_embed or its gradient is present; compact: the plan with the
-// smallest workspace instead of the fastest).
-void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool compact);
+// n_chunks / n_tiles_kv (se: scale_embed or its gradient is present; dg: the score gain's gradient is
+// requested; compact: the plan with the smallest workspace instead of the fastest).
+void bwd_plan(BwdParams& p, int D, int dtype, bool se, bool dg, bool compact);
 
 // bf16 MFMA backward kernels: same conditions as the MFMA forward.
 bool bwd_mfma_supported(const BwdParams& p, int D, int dtype);
+// Workgroups of the scale_embed dq that a CU holds, with ns long-range taps.
+int bwd_dq_se_resident(int D, int ns, bool dg);
 hipError_t launch_bwd_dq_mfma(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
 hipError_t launch_bwd_dkdv_mfma(const BwdParams& p, int D, unsigned nblocks, hipStream_t st);
 hipError_t launch_bwd_reduce(const ReduceParams& r, hipStream_t st);
