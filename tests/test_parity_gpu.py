@@ -225,8 +225,8 @@ def test_heads_without_scale_embed(gpu_device, D, offsets, gains):
 @pytest.mark.parametrize("offsets", [OFFSETS_J46, OFFSETS_J47], ids=["J46", "J47"])
 def test_score_gain_gradient_with_scale_embed(gpu_device, D, offsets):
     """scale_embed with both gains over the 46- and 47-offset tables at D = 32 and 64: dq's
-    score-gain gradient forms with scale_embed for 13 and 14 long-range taps (two batches, so
-    a batch group sums two slices)."""
+    score-gain gradient forms with scale_embed for 13 and 14 long-range taps, one batch per
+    workgroup (groups of batches: tests/test_bwd_batches.py)."""
     inp = _rand_inputs(2, 3, 1100, D, offsets, torch.bfloat16, seed=700 + D + len(offsets))
     _say(f"bf16 B2 H3 N1100 D{D} J{len(offsets)} with se, g, a")
     got = gpu_run(inp, offsets, gpu_device)
@@ -237,10 +237,10 @@ def test_score_gain_gradient_with_scale_embed(gpu_device, D, offsets):
 @pytest.mark.parametrize("gains", [True, False])
 @pytest.mark.parametrize("B", [3, 5, 6])
 def test_scale_embed_batch_groups(gpu_device, B, gains):
-    """With scale_embed the dq workgroup takes one head and tile in four batches and sums its
-    parameter partials over them; batch counts that leave a short last group (or one group of
-    three) against the oracle, with the score gain's gradient (the generic dq) and without it
-    (the 11-tap dq of the reference modules' call)."""
+    """With scale_embed the dq workgroup takes one head and tile in one, two or four batches, by how
+    its grid fills the chip: odd and even batch counts of a grid that takes one batch each, against
+    the oracle, with the score gain's gradient and without it (the reference modules' call).
+    Groups of two and four, with short last ones: tests/test_bwd_batches.py."""
     inp = _rand_inputs(B, 3, 700, 64, OFFSETS_V3, torch.bfloat16, seed=300 + B, gains=gains)
     _say(f"bf16 B{B} H3 N700 D64 with se, gains={gains} (batch groups)")
     got = gpu_run(inp, OFFSETS_V3, gpu_device)
