@@ -69,10 +69,14 @@ template <> struct Vec8<bf16_t> {
 // Raw 16-byte chunk copy (8 bf16 or 4 f32), used to stage rows into LDS unchanged.
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ void st16(void* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
-// 16 bytes stored past the caches' retention (a non-temporal store), for results that nothing in
-// this launch or the next reads: kept in L2 they push out the rows that the long-range taps gather
-// again (a forward + backward at B4 H8 N4096 D64: dk/dv 44 -> 32 us, dq 49 -> 43; B8 H8 N2048 D96
-// with scale_embed: forward 52 -> 43).
+// 16 bytes stored past the caches' retention (a non-temporal store), for results that neither this
+// launch nor the attention's next one reads: kept in L2 they push out the rows that the long-range
+// taps gather again (a forward + backward at B4 H8 N4096 D64: dk/dv 44 -> 32 us, dq 49 -> 43; B8 H8
+// N2048 D96 with scale_embed: forward 52 -> 43).  In a module the launch after the forward, the gate
+// product, does read out, and the projection's backward d(qkv): its step is as fast or faster all
+// the same (bf16 B8 N2048: E 768 H 12 686 -> 678 us, E 768 H 8 702 -> 697, E 256 H 8 478 -> 481),
+// and the forward with the gate product is, but at D = 80 (B4 H8 N2047 28.1 -> 29.4 us, where forward
+// + backward gains as much: 72.6 -> 71.0).
 __device__ __forceinline__ void st16_stream(void* p, uint4 v) {
   typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(p));

@@ -646,9 +646,18 @@ Tensor pool_gate(const Tensor& x, const Tensor& g) {
 
 // Whether the weight gradient goes to dsqg_linear_wgrad: 16-bit operands of aligned widths, and an
 // output small enough that the library's tiling of it alone leaves most of the chip idle.  Against
-// its product and column sum (us, 16-bit, rows x O x I): 512 x 256 x 256 12 / 40,
-// 16384 x 256 x 256 17 / 122, 16384 x 768 x 768 50 / 124, 16384 x 3072 x 768 157 / 224,
-// 65536 x 2304 x 768 430 / 609; 65536 x 3072 x 768 578 / 548.
+// its product and column sum, both callers' host time included (us, either type), by O x I and rows:
+//                 512      2048      4096       16384      32768       65536
+//   256 x 256   9 / 29   10 / 27   11 / 41    18 / 114    17 / 139    24 / 242
+//   768 x 768  12 / 27   20 / 29   24 / 46    45 / 114    79 / 212   145 / 308
+//  1024 x 2048 20 / 27   25 / 34   37 / 55   112 / 145   214 / 321   500 / 573
+//  1536 x 1536 21 / 29   29 / 42   44 / 64   144 / 178   277 / 330   562 / 596
+//  3072 x 768  21 / 27   29 / 42   44 / 60   143 / 178   277 / 327   571 / 514
+//  1792 x 1792 24 / 29   32 / 44   51 / 64   162 / 176   312 / 345   621 / 660
+//  2048 x 2048 25 / 27   40 / 44   65 / 62   215 / 180   468 / 318   965 / 604
+// The library's time depends on the shape where the two are close, so the lines lie inside: up to
+// 2^21 outputs, where every measured row count wins by an eighth or more, and up to 3072 x 768, the
+// widest layer of the reference's models, for the rows at which every such shape wins by a seventh.
 bool use_wgrad(at::ScalarType dt, int64_t T, int64_t O, int64_t I) {
   if ((dt != at::kHalf && dt != at::kBFloat16) || T < 1 || O < 1 || O % 8 != 0 || I % 8 != 0) return false;
   if ((T + 128) * std::max(O, I) * 2 >= (1ll << 31)) return false;

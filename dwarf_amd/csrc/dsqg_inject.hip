@@ -52,8 +52,8 @@ __device__ __forceinline__ void store8(void* base, long long e, const float (&x)
   else Vec8<bf16_t>::store(static_cast<bf16_t*>(base) + e, x);
 }
 
-// DT: type of qkv; KDT: of both deltas; ODT: of the outputs.
-template <int DT, int KDT, int ODT>
+// DT: type of qkv and of both deltas; ODT: of the outputs.
+template <int DT, int ODT>
 __global__ __launch_bounds__(kBlock) void kv_inject_kernel(InjectParams p) {
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (t >= p.pieces) return;
@@ -65,11 +65,11 @@ __global__ __launch_bounds__(kBlock) void kv_inject_kernel(InjectParams p) {
   float k[8], v[8], kd[8], vd[8], q[8];
   load8<DT>(p.qkv, src + E, k);
   load8<DT>(p.qkv, src + 2 * E, v);
-  load8<KDT>(p.kd, b * p.kb + h * p.kh + n * p.kn + d, kd);
-  load8<KDT>(p.vd, b * p.vb + h * p.vh + n * p.vn + d, vd);
+  load8<DT>(p.kd, b * p.kb + h * p.kh + n * p.kn + d, kd);
+  load8<DT>(p.vd, b * p.vb + h * p.vh + n * p.vn + d, vd);
   if (p.q_out) load8<DT>(p.qkv, src, q);
   round8<DT, ODT>(k); round8<DT, ODT>(v);
-  round8<KDT, ODT>(kd); round8<KDT, ODT>(vd);
+  round8<DT, ODT>(kd); round8<DT, ODT>(vd);
 #pragma unroll
   for (int i = 0; i < 8; ++i) { k[i] += kd[i]; v[i] += vd[i]; }
   store8<ODT>(p.k_out, dst, k);
@@ -77,9 +77,9 @@ __global__ __launch_bounds__(kBlock) void kv_inject_kernel(InjectParams p) {
   if (p.q_out) store8<ODT>(p.q_out, dst, q);
 }
 
-template <int DT, int KDT, int ODT>
+template <int DT, int ODT>
 void launch(const InjectParams& p, hipStream_t st) {
-  hipLaunchKernelGGL((kv_inject_kernel<DT, KDT, ODT>), dim3((unsigned)((p.pieces + kBlock - 1) / kBlock)), dim3(kBlock),
+  hipLaunchKernelGGL((kv_inject_kernel<DT, ODT>), dim3((unsigned)((p.pieces + kBlock - 1) / kBlock)), dim3(kBlock),
                      0, st, p);
 }
 
@@ -115,13 +115,11 @@ extern "C" int dsqg_kv_inject(const dsqg_kv_inject_args* a, dsqg_stream_t stream
   p.pieces = (long long)a->B * a->N * p.E8;
   if (p.pieces > (1ll << 31)) return DSQG_EUNSUPPORTED;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // The combinations the host layer makes: operands of the output type, and float16 to bf16.
-  const int key = a->qkv_dtype * 16 + a->delta_dtype * 4 + a->out_dtype;
-  switch (key) {
-    case DSQG_F32 * 16 + DSQG_F32 * 4 + DSQG_F32: launch<DSQG_F32, DSQG_F32, DSQG_F32>(p, st); break;
-    case DSQG_BF16 * 16 + DSQG_BF16 * 4 + DSQG_BF16: launch<DSQG_BF16, DSQG_BF16, DSQG_BF16>(p, st); break;
-    case DSQG_F16 * 16 + DSQG_F16 * 4 + DSQG_BF16: launch<DSQG_F16, DSQG_F16, DSQG_BF16>(p, st); break;
-    default: return DSQG_EUNSUPPORTED;
-  }
+  // What the host layer asks for: operands of the output type, and float16 to bf16.
+  if (a->delta_dtype != a->qkv_dtype) return DSQG_EUNSUPPORTED;
+  if (a->qkv_dtype == DSQG_F32 && a->out_dtype == DSQG_F32) launch<DSQG_F32, DSQG_F32>(p, st);
+  else if (a->qkv_dtype == DSQG_BF16 && a->out_dtype == DSQG_BF16) launch<DSQG_BF16, DSQG_BF16>(p, st);
+  else if (a->qkv_dtype == DSQG_F16 && a->out_dtype == DSQG_BF16) launch<DSQG_F16, DSQG_BF16>(p, st);
+  else return DSQG_EUNSUPPORTED;
   return hipGetLastError() == hipSuccess ? DSQG_OK : DSQG_EHIP;
 }

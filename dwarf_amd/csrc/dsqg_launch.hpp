@@ -9,8 +9,8 @@ namespace dsqg {
 // hipErrorInvalidValue for a head dim without a kernel (the ABI checks that first).
 hipError_t launch_fwd(const FwdParams& p, int dtype, int D, hipStream_t st);
 
-// bf16 MFMA forward (dsqg_fwd_mfma.hip): head dims 32/64/128, at most kMaxSparse taps beyond
-// the dense window, row strides >= D and 32-bit byte offsets within each (b,h) slice.
+// bf16 MFMA forward (dsqg_fwd_mfma.hip): every head dim, at most kMaxSparse taps beyond the dense
+// window, row strides >= D and 32-bit byte offsets within each (b,h) slice.
 // launch_fwd picks it whenever it applies.
 bool fwd_mfma_supported(const FwdParams& p, int D);
 hipError_t launch_fwd_mfma(const FwdParams& p, int D, hipStream_t st);
