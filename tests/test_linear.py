@@ -31,15 +31,27 @@ def _close(got, dy, x, name):
     (1, 8, 8, 0), (63, 8, 136, 8), (64, 128, 128, 0), (65, 136, 120, 0), (256, 256, 128, 24),
     (257, 128, 264, 0), (1000, 264, 520, 0), (8191, 256, 256, 0), (70001, 8, 8, 0)])
 def test_kernel_against_float64(gpu_device, T, O, I, pad, dtype):
+    _run_kernel(gpu_device, T, O, I, pad, dtype, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 200, 256, 257])  # one split, straight to the results; two
+def test_float32_results_against_float64(gpu_device, T, dtype):
+    _run_kernel(gpu_device, T, 136, 264, 8, dtype, torch.float32)
+
+
+def _run_kernel(gpu_device, T, O, I, pad, dtype, out):
+    code = {torch.float16: _lib.DSQG_F16, torch.bfloat16: _lib.DSQG_BF16, torch.float32: _lib.DSQG_F32}
     g = torch.Generator().manual_seed(T + O + I)
     dy = torch.randn(T, O + pad, generator=g).to(gpu_device, dtype)[:, :O]
     x = torch.randn(T, I + pad, generator=g).to(gpu_device, dtype)[:, :I]
     a = _lib.LinearWgradArgs()
     a.T, a.O, a.I = T, O, I
-    a.dtype = a.out_dtype = _lib.DSQG_F16 if dtype == torch.float16 else _lib.DSQG_BF16
+    a.dtype, a.out_dtype = code[dtype], code[out]
     a.dy, a.dy_stride, a.x, a.x_stride = dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0)
-    dw = torch.full((O, I), float("nan"), device=gpu_device, dtype=dtype)
-    db = torch.full((O,), float("nan"), device=gpu_device, dtype=dtype)
+    dw = torch.full((O, I), float("nan"), device=gpu_device, dtype=out)
+    db = torch.full((O,), float("nan"), device=gpu_device, dtype=out)
     a.dw, a.db = dw.data_ptr(), db.data_ptr()
     n = ctypes.c_size_t(0)
     lib = _lib.load()
