@@ -411,13 +411,13 @@ struct AttentionQkvKvFunction : torch::autograd::Function<AttentionQkvKvFunction
 
 // The per-tap and per-head parameters for H heads of HD over the table t (the kernels index them by these).
 void check_params(const Params& P, int64_t H, int64_t HD, const Table& t) {
-  auto expect = [](const Tensor& x, std::vector<int64_t> s, const char* name) {
-    if (x.defined() && x.sizes() != c10::IntArrayRef(s))
-      require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
+  const int64_t J = t.J;
+  auto expect = [](const Tensor& x, c10::IntArrayRef s, const char* name) {
+    if (x.defined() && x.sizes() != s) require(false, name, " must be ", shape_str(s), ", got ", shape_str(x.sizes()));
   };
-  expect(P.pb, {t.J, H}, "pos_bias");
-  expect(P.se, {t.J, HD}, "scale_embed");
-  expect(P.sg, {H, t.J}, "score_gain");
+  expect(P.pb, {J, H}, "pos_bias");
+  expect(P.se, {J, HD}, "scale_embed");
+  expect(P.sg, {H, J}, "score_gain");
   expect(P.ig, {H}, "if_gain");
 }
 
@@ -480,8 +480,10 @@ Tensor decode(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor
   py::gil_scoped_release nogil;
   require(k_ring.dim() == 4, "k_ring must be [B,H,S,D], got ", shape_str(k_ring.sizes()));
   check_params({pb0, undef(se0), undef(sg0), undef(ig0)}, k_ring.size(1), k_ring.size(3), *t);
-  auto f32 = [](const Tensor& x) { return x.defined() ? x.detach().to(at::kFloat).contiguous() : x; };
-  const Tensor q = q0.contiguous(), k = k0.contiguous(), v = v0.contiguous();
+  // (The kernel reads stored values: lazily negated operands are resolved, as the op's dispatch does.)
+  auto ready = [](const Tensor& x) { return x.is_neg() ? x.resolve_neg().contiguous() : x.contiguous(); };
+  auto f32 = [&](const Tensor& x) { return x.defined() ? ready(x.detach().to(at::kFloat)) : x; };
+  const Tensor q = ready(q0), k = ready(k0), v = ready(v0);
   const Tensor pos = pos0.to(at::kLong).contiguous();
   const Tensor pb = f32(pb0), se = f32(undef(se0)), sg = f32(undef(sg0)), ig = f32(undef(ig0));
   const Tensor out = at::empty_like(q);

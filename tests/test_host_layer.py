@@ -160,6 +160,18 @@ def test_decode_marks_the_rings_changed(gpu_device):
         dwarf_amd.dsqg_decode_step(rows[0].requires_grad_(True), *rows[1:], *rings, pos, pb).float().sum().backward()
 
 
+@gpu
+def test_decode_of_lazily_negated_operands(gpu_device):
+    rows = [torch.randn(B, H, D, device=gpu_device).bfloat16() for _ in range(3)]
+    pos, pb = torch.tensor([3, 2000], device=gpu_device), torch.randn(44, H, device=gpu_device)
+    rings = torch.randn(2, B, H, 1537, D, device=gpu_device).bfloat16()
+    res = []
+    for args in ([torch._neg_view(t) for t in (*rows, pb)], [-t for t in (*rows, pb)]):
+        kr, vr = rings.clone()
+        res.append((dwarf_amd.dsqg_decode_step(*args[:3], kr, vr, pos, args[3]), kr, vr))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
 class _NoGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
